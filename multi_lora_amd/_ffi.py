@@ -204,6 +204,35 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+# Order of the addresses _calls.set_library takes.
+_CALLS_FUNCTIONS = ("mlora_last_error", "mlora_shrink_workspace_bytes", "mlora_shrink", "mlora_expand",
+                    "mlora_apply_segments_workspace_bytes", "mlora_apply_segments", "mlora_rmsnorm",
+                    "mlora_add_rmsnorm", "mlora_grouped_workspace_bytes", "mlora_apply_grouped",
+                    "mlora_rmsnorm_apply_grouped")
+_calls_module = None
+
+
+def calls():
+    """The native form of the entry points' ordinary calls (csrc/host/calls.cpp),
+    given the loaded library; raises if it is not built."""
+    global _calls_module
+    if _calls_module is not None:
+        return _calls_module
+    handle = lib()
+    with _lock:
+        if _calls_module is None:
+            from .batch_info import PLAN_LONG_ROWS, KernelInputMetaData
+            try:
+                from . import _calls as module
+            except ImportError as e:
+                raise RuntimeError(f"{LIB_PATH.parent / '_calls.so'} is not built ({e}); run "
+                                   "`python -m multi_lora_amd.build`") from e
+            module.set_library(tuple(ctypes.cast(getattr(handle, f), ctypes.c_void_p).value for f in _CALLS_FUNCTIONS),
+                               MloraError, KernelInputMetaData, PLAN_LONG_ROWS)
+            _calls_module = module
+    return _calls_module
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODE[dtype]

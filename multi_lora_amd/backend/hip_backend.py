@@ -16,6 +16,7 @@ from typing import Callable, List, Optional, Sequence
 
 import torch
 
+from .. import _ffi
 from ..kernels.lora_ops import (GROUPED_MAX_LEN, LinkedWorkspace, Workspace, apply_grouped, apply_segments, expand,
                                  planned_pays, reserve_segments, rmsnorm_apply_grouped, shrink)
 from ..kernels.rmsnorm import rmsnorm_fwd
@@ -79,6 +80,11 @@ class HipLoRABackend(LoRABackend):
         Equal to ``apply_lora`` per slice on the column views, element for element.
         """
         meta = self._meta()
+        # The ordinary call, checked and launched natively; what it does not
+        # take (None) runs, or raises, below.
+        if _ffi.calls().apply_multi(x, a_stacks, b_stacks, meta, base_output, col_offsets, self.linked_workspace,
+                                    self.workspace):
+            return base_output
         if x.dim() != 2:
             raise ValueError("HipLoRABackend expects x [S, in]")
         if col_offsets is None:
@@ -131,10 +137,14 @@ class HipLoRABackend(LoRABackend):
         b_stacks = [b.contiguous() for b in b_stacks]
         y = torch.empty_like(x)
         args = (x, weight, eps, y, a_stacks, b_stacks, meta, base_output, col_offsets, self.linked_workspace)
-        if meta.max_len <= GROUPED_MAX_LEN and rmsnorm_apply_grouped(*args, phases=1):
+
+        def fused(phases: int) -> bool:
+            return bool(_ffi.calls().rmsnorm_apply(*args, phases)) or rmsnorm_apply_grouped(*args, phases=phases)
+
+        if meta.max_len <= GROUPED_MAX_LEN and fused(3 if base_fn is None else 1):
             if base_fn is not None:
                 base_fn(y, base_output)
-            rmsnorm_apply_grouped(*args, phases=2)
+                fused(2)
             return y
         y = rmsnorm_fwd(x, weight, eps)
         if base_fn is not None:

@@ -25,6 +25,8 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libmlora_hip.so"
 CALIB_LIB = PKG / "libmlora_calib.so"
+CALLS_SRC = CSRC / "host" / "calls.cpp"
+CALLS_MODULE = PKG / "_calls.so"
 ARCH = os.environ.get("MLORA_OFFLOAD_ARCH", "gfx950")
 
 HIP_FLAGS = [
@@ -80,9 +82,31 @@ def _link(objs, lib: Path) -> None:
     os.replace(tmp, lib)
 
 
+def _build_calls(_=None) -> None:
+    """The CPython extension of csrc/host/calls.cpp (host code: g++ against torch's headers and libraries)."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    tmp = CALLS_MODULE.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-isystem{d}" for d in (root / "include", root / "include/torch/csrc/api/include", rocm / "include",
+                                      sysconfig.get_paths()["include"])),
+           str(CALLS_SRC), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10",
+           "-lc10_hip", "-lamdhip64"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {CALLS_SRC.name}:\n{proc.stderr}")
+    os.replace(tmp, CALLS_MODULE)
+
+
 def build(verbose: bool = True) -> Path:
     """Compile every HIP source, link the product library and the
-    measurement library; returns the product library's path."""
+    measurement library, and build the native call module; returns the
+    product library's path."""
     cal_dir = BUILD / "calib"
     cal_dir.mkdir(parents=True, exist_ok=True)
     srcs = sources()
@@ -90,7 +114,9 @@ def build(verbose: bool = True) -> Path:
     cal_jobs = [(s, cal_dir / (s.stem + ".o"), ["-DMLORA_TIMELINE=1"]) for s in srcs + calib_sources()]
     workers = min(len(jobs) + len(cal_jobs), int(os.environ.get("MAX_JOBS", "8")), 16)
     with ThreadPoolExecutor(max_workers=max(1, workers)) as pool:
+        calls = pool.submit(_build_calls)
         objs = list(pool.map(_compile, jobs + cal_jobs))
+        calls.result()
     _link(objs[:len(jobs)], LIB)
     _link(objs[len(jobs):], CALIB_LIB)
     if verbose:

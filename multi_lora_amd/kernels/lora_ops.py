@@ -24,7 +24,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 
 from .. import _ffi
-from ..batch_info import PLAN_LONG_ROWS, KernelInputMetaData
+from ..batch_info import KernelInputMetaData
 
 _WORKSPACES: Dict[Tuple[str, int], torch.Tensor] = {}
 
@@ -60,10 +60,10 @@ class LinkedWorkspace:
     """
 
     def __init__(self) -> None:
-        self.bufs: Dict[Tuple[torch.device, int], torch.Tensor] = {}
+        self.bufs: Dict[Tuple[int, int], torch.Tensor] = {}  # by (device index, stream handle)
 
     def get(self, nbytes: int, device: torch.device, stream: int) -> Tuple[int, int]:
-        key = (device, stream)
+        key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
         buf = self.bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
@@ -259,11 +259,6 @@ def expand(mid: torch.Tensor, b_stacks: Sequence[torch.Tensor], meta: KernelInpu
 GROUPED_MAX_LEN = 16
 
 
-# Bytes of adapter and row tiles the planned path's work items may read in all
-# for a batch with segments of more than 16 rows (planned_pays).
-PLANNED_LONG_BYTES = 56 << 20
-
-
 def planned_pays(meta: KernelInputMetaData, x: torch.Tensor, a_stacks: Sequence[torch.Tensor],
                  b_stacks: Sequence[torch.Tensor]) -> bool:
     """Whether a batch with segments of more than 16 rows runs faster through
@@ -279,22 +274,10 @@ def planned_pays(meta: KernelInputMetaData, x: torch.Tensor, a_stacks: Sequence[
     400 rows at rank 64 (35 MB) 11.7 vs 16.0; 800 rows at rank 16 (32 MB)
     10.7 vs 14.2, at rank 64 (70 MB) 20.2 vs 19.0; 1600 rows at rank 16
     (64 MB) 18.1 vs 17.5; 1088 mixed rows to 6144 columns (108 MB) 27.2 vs
-    24.3.  Captured calls stay with the segment path, which reads the table
+    24.3; the line is drawn at 56 MB.  Captured calls stay with the segment path, which reads the table
     itself: a replay follows every rewrite of it.
     """
-    # The cheap tests first: most prompt batches end here.
-    if x.shape[0] > PLAN_LONG_ROWS:
-        return False
-    n, shape = len(a_stacks), a_stacks[0].shape
-    if len(shape) != 3 or getattr(meta, "packed", None) is None:
-        return False
-    r_max = shape[1]
-    cost = ((x.shape[1] + 255) >> 8) * (16 * (1 if n * r_max <= 64 else n) + n * r_max)
-    for b in b_stacks:
-        cost += ((b.shape[1] + 255) >> 8) * (r_max + 32)
-    if meta.plan_entries * cost * 512 > PLANNED_LONG_BYTES:
-        return False
-    return meta.plan_is_current(x.shape[0]) and not torch.cuda.is_current_stream_capturing()
+    return bool(_ffi.calls().planned_pays(meta, x, a_stacks, b_stacks))
 
 
 class _DevicePlan:
@@ -555,6 +538,9 @@ def sgemm_lora_a_fwd(x: torch.Tensor, weights: torch.Tensor, kernel_input_metada
     x: ``[S, in]``, weights: ``[K, r_max, in]``, output: a caller-owned
     ``[>=S, >=r_max]`` buffer; returns the ``[S, r_max]`` view written.
     """
+    out = _ffi.calls().sgemm_a(x, weights, kernel_input_metadata, output, stack_num, _WORKSPACES)
+    if out is not None:
+        return out
     assert x.is_contiguous()
     assert weights.is_contiguous()
     assert len(x.shape) == 2
@@ -573,6 +559,8 @@ def sgemm_lora_b_fwd(x: torch.Tensor, weights: torch.Tensor, kernel_input_metada
     x (mid): ``[S, r_max]``, weights: ``[K, out, r_max]``.  With
     ``base_output=None`` a zero output is allocated and returned.
     """
+    if base_output is not None and _ffi.calls().sgemm_b(x, weights, kernel_input_metadata, base_output):
+        return base_output
     assert x.is_contiguous()
     assert weights.is_contiguous()
     assert len(x.shape) == 2

@@ -17,6 +17,9 @@ from .. import _ffi
 
 def rmsnorm_fwd(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``x * rsqrt(mean(x^2, -1) + eps) * weight`` in fp32, rounded once to x.dtype."""
+    out = _ffi.calls().rmsnorm(x, weight, eps) if x.is_cuda else None
+    if out is not None:
+        return out
     if x.device.type != "cuda":
         raise RuntimeError(f"x must be on a ROCm GPU (got {x.device}); the HIP path has no CPU fallback")
     hidden = x.shape[-1]
@@ -56,6 +59,9 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
     (OPTIMIZATION_TODO.md T22).  Returns the normalised rows (a new tensor);
     ``residual`` holds ``x + residual`` afterwards.
     """
+    out = _ffi.calls().add_rmsnorm(x, residual, weight, eps) if x.is_cuda else None
+    if out is not None:
+        return out
     if x.device.type != "cuda":
         raise RuntimeError(f"x must be on a ROCm GPU (got {x.device}); the HIP path has no CPU fallback")
     hidden = x.shape[-1]
