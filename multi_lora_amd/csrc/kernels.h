@@ -199,7 +199,8 @@ struct DecodeArgs {
   int s_groups;      // shrink items per (entry, chunk): 1 (all slices) or n_slices (one each)
   int n_tiles;       // expand items per entry (256-column tiles over all slices)
   int tile_base[kMaxSlices + 1];
-  int e_grid;        // entries per row of the grid (multiple of 8)
+  int e_grid;        // entries the grid holds (multiple of 8)
+  int item_fast;     // grid order: an entry's items next to each other (x), else the entries
   int e_cap;         // entries the workspace flags hold
   int plan_cap;      // entries the plan holds
   int ws_rows;       // rows the workspace sums hold

@@ -550,3 +550,32 @@ def test_largest_supported_shape(dev):
     lws.set_wait_ticks(-1)
     assert torch.equal(grouped(wl, mode=1, lws=lws), one)
     assert counters(lws)[0] > 0
+
+
+@pytest.mark.parametrize("in_dim,out,r_max,ranks", [
+    (4104, 264, 64, [64, 33, 8, 16]),    # last K chunk of one 16-byte piece, a ragged column tile
+    (2552, 512, 40, [40, 13]),           # B rows of five pieces
+    (4096, 768, 24, [24, 8, 17]),
+])
+def test_large_two_launch_grids_equal_the_single_launch(dev, in_dim, out, r_max, ranks):
+    """Grids of more than 1024 shrink items (staged rows, an entry's items next
+    to each other) against the single launch, bit for bit, and the oracle."""
+    n_slots, rows = 130, 200
+    g = torch.Generator().manual_seed(in_dim)
+    slots = [i % n_slots for i in range(rows)]
+    slot_ranks = [ranks[i % len(ranks)] for i in range(n_slots)]
+    x = torch.randn(rows, in_dim, generator=g).bfloat16()
+    a = (torch.randn(n_slots, r_max, in_dim, generator=g) * in_dim ** -0.5).bfloat16()
+    b = (torch.randn(n_slots, out, r_max, generator=g) * 0.05).bfloat16()
+    base = torch.randn(rows, out, generator=g).bfloat16()
+    scal = [0.5 + (i % 3) for i in range(n_slots)]
+    meta = make_meta([1] * rows, slots, slot_ranks, scal, dev, torch.bfloat16)
+    assert meta.plan_entries * -(-in_dim // 256) > 1024
+    outs = []
+    for mode in (1, 2):
+        got = base.to(dev)
+        assert apply_grouped(x.to(dev), [a.to(dev)], [b.to(dev)], meta, got, [0], LinkedWorkspace(), mode=mode)
+        outs.append(got.cpu())
+    assert torch.equal(outs[0], outs[1])
+    assert_tol_f64(outs[0], apply_f64(x, [a], [b], make_meta([1] * rows, slots, slot_ranks, scal, "cpu",
+                                                             torch.bfloat16), base, [0]))
