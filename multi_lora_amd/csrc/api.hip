@@ -94,6 +94,16 @@ size_t mid_region_bytes(int32_t rows, int32_t n_slices, int32_t r_max, int32_t d
   return (b + 255) / 256 * 256;
 }
 
+// Whether every row the shrink reads is made of 16-byte chunks.
+bool shrink_aligned(const void* x, int64_t x_row_stride, int32_t in_dim, const mlora_slice* slices, int32_t n_slices,
+                    int32_t dtype) {
+  const int vec = vec_elems(dtype);
+  bool aligned = al16(x) && x_row_stride % vec == 0 && in_dim % vec == 0;
+  for (int s = 0; s < n_slices; ++s)
+    aligned = aligned && al16(slices[s].a) && slices[s].a_slot_stride % vec == 0 && slices[s].a_row_stride % vec == 0;
+  return aligned;
+}
+
 // Shrink; with skip_reduce the split sums stay in the workspace for the
 // expand (no reduce launch).  private_mid: only the apply path's expand
 // reads mid, so the split reduce may fill every row and column of it
@@ -120,17 +130,13 @@ int shrink_impl(const void* x, int64_t x_row_stride, int32_t num_rows, int32_t i
                   (long long)slices[s].a_slot_stride, (long long)slices[s].a_row_stride, r_max, in_dim);
   }
 
+  const bool aligned = shrink_aligned(x, x_row_stride, in_dim, slices, n_slices, dtype);
   mlora::ShrinkPlan plan;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, meta->bs, meta->max_len, dtype, num_cus(), &plan))
+  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, meta->bs, meta->max_len, dtype, aligned, num_cus(), &plan))
     return fail(kUnsupported, "shrink shape unsupported: %d slices x r_max %d exceeds 16 blocks of 16 rows",
                 n_slices, r_max);
   if (plan.ws_bytes > 0 && (workspace == nullptr || workspace_bytes < plan.ws_bytes))
     return fail(kWorkspace, "shrink workspace too small: need %zu bytes, got %zu", plan.ws_bytes, workspace_bytes);
-
-  const int vec = vec_elems(dtype);
-  bool aligned = al16(x) && x_row_stride % vec == 0 && in_dim % vec == 0;
-  for (int s = 0; s < n_slices; ++s)
-    aligned = aligned && al16(slices[s].a) && slices[s].a_slot_stride % vec == 0 && slices[s].a_row_stride % vec == 0;
 
   mlora::ShrinkArgs args{};
   args.x = x;
@@ -235,7 +241,7 @@ size_t mlora_shrink_workspace_bytes(int32_t in_dim, int32_t r_max, int32_t n_sli
                                     int32_t max_len, int32_t dtype) {
   if (!valid_dtype(dtype)) return 0;
   mlora::ShrinkPlan p;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, num_cus(), &p)) return 0;
+  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, true, num_cus(), &p)) return 0;
   return p.ws_bytes;
 }
 
@@ -260,7 +266,7 @@ size_t mlora_apply_segments_workspace_bytes(int32_t in_dim, int32_t r_max, int32
                                             int32_t bs, int32_t max_len, int32_t dtype) {
   if (!valid_dtype(dtype) || num_rows < 0 || r_max <= 0 || n_slices < 1) return 0;
   mlora::ShrinkPlan p;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, num_cus(), &p)) return 0;
+  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, true, num_cus(), &p)) return 0;
   return mid_region_bytes(num_rows, n_slices, r_max, dtype) + p.ws_bytes;
 }
 
@@ -274,8 +280,9 @@ int mlora_apply_segments(const void* x, int64_t x_row_stride, int32_t num_rows, 
   if (n_slices < 1 || n_slices > MLORA_MAX_SLICES) return fail(kBadArg, "n_slices %d not in [1, %d]", n_slices, MLORA_MAX_SLICES);
   if (in_dim <= 0 || r_max <= 0 || num_rows < 0) return fail(kBadArg, "in_dim %d, r_max %d, num_rows %d", in_dim, r_max, num_rows);
   if (meta->bs == 0 || num_rows == 0) return 0;
+  const bool aligned = slices != nullptr && shrink_aligned(x, x_row_stride, in_dim, slices, n_slices, dtype);
   mlora::ShrinkPlan plan;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, meta->bs, meta->max_len, dtype, num_cus(), &plan))
+  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, meta->bs, meta->max_len, dtype, aligned, num_cus(), &plan))
     return fail(kUnsupported, "shrink shape unsupported: %d slices x r_max %d exceeds 16 blocks of 16 rows",
                 n_slices, r_max);
   const size_t mid_bytes = mid_region_bytes(num_rows, n_slices, r_max, dtype);

@@ -55,13 +55,19 @@ struct ShrinkPlan {
   int spg;        // slices per launch: calls over 8 A blocks run one launch per group of slices
   int kt;         // streamed kernel: reduction elements per stage (0: not planned)
   int stages;     // streamed kernel: stages in flight
+  int wide;       // whole reduction per workgroup (shrink_wide.hip): 16-row tiles, ks 1
   size_t ws_bytes;
 };
 
-bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, int num_cus,
-                 ShrinkPlan* plan);
+// aligned: every operand row is readable as 16-byte chunks.  A plan of
+// unaligned rows needs no more workspace than the aligned one.
+bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, bool aligned,
+                 int num_cus, ShrinkPlan* plan);
 // Launches the shrink and, when K is split, the in-order split reduction.
 hipError_t launch_shrink(const ShrinkPlan& plan, ShrinkArgs args, int dtype, bool aligned, hipStream_t stream);
+
+// The shrink without a K split (a plan with `wide` set; args complete).
+hipError_t launch_shrink_wide(const ShrinkPlan& plan, const ShrinkArgs& args, int dtype, bool aligned, hipStream_t stream);
 
 // -------------------------------------------------------------- expand
 constexpr int kExpandBN = 256;  // output columns per tile

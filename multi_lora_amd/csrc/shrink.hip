@@ -13,12 +13,14 @@
 //   short segments (<= 16 rows, shrink_kernel): workgroup = (segment, K
 //     split); the 4 waves take alternate K-steps of the same 16 rows and are
 //     summed through LDS in wave order.
+//   calls whose tiles are few or small, unaligned 16-bit rows, most fp32:
+//     workgroup = 16-row tile over the whole reduction (shrink_wide.hip).
 //   long segments: workgroup = (dense 64-row tile, K split); each wave owns
 //     16 rows of the tile and every rank block.  16-bit aligned data with K
 //     splits in multiples of 64 stream x and A straight into LDS three
 //     stages deep (shrink_dma_kernel); other 16-bit aligned data stage them
-//     through registers (shrink_lds_kernel); the rest load MFMA fragments
-//     directly (shrink_rows_kernel).
+//     through registers (shrink_lds_kernel); fp32 and more than eight A
+//     blocks load MFMA fragments directly (shrink_rows_kernel).
 // When K is split over workgroups each split stores fp32 sums and a second
 // launch adds them in split order, so the result is deterministic and no
 // workgroup ever waits on another.
@@ -26,6 +28,8 @@
 // Loads in the K loop are unconditional: rows past the segment end or the
 // rank are clamped to a row that exists (their products are discarded), so a
 // wave keeps several 16-byte loads of x and A in flight.
+#include <algorithm>
+
 #include "kernels.h"
 #include "loads.h"
 
@@ -828,7 +832,9 @@ hipError_t launch_nbt_al(const ShrinkPlan& p, const ShrinkArgs& args, hipStream_
   if (p.bm != 64 * RB) return hipErrorInvalidValue;
   if constexpr (AL && sizeof(typename T::raw_t) == 2 && NBT <= 8)
     return launch_with<T>(shrink_lds_kernel<T, NBT, RB>, p, args, stream);
-  return launch_with<T>(shrink_rows_kernel<T, NBT, RB, AL>, p, args, stream);
+  // Unaligned 16-bit rows of up to eight blocks are the wide kernel's.
+  if constexpr (!AL && sizeof(typename T::raw_t) == 2 && NBT <= 8) return hipErrorInvalidValue;
+  else return launch_with<T>(shrink_rows_kernel<T, NBT, RB, AL>, p, args, stream);
 }
 
 template <class T, bool AL>
@@ -843,9 +849,14 @@ hipError_t launch_al(const ShrinkPlan& p, const ShrinkArgs& args, hipStream_t st
 }
 
 template <class T>
-hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, bool aligned, hipStream_t stream) {
-  if (p.spg >= args.n_slices)
-    return aligned ? launch_al<T, true>(p, args, stream) : launch_al<T, false>(p, args, stream);
+hipError_t launch_group(const ShrinkPlan& p, const ShrinkArgs& args, int dtype, bool aligned, hipStream_t stream) {
+  if (p.wide) return launch_shrink_wide(p, args, dtype, aligned, stream);
+  return aligned ? launch_al<T, true>(p, args, stream) : launch_al<T, false>(p, args, stream);
+}
+
+template <class T>
+hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, int dtype, bool aligned, hipStream_t stream) {
+  if (p.spg >= args.n_slices) return launch_group<T>(p, args, dtype, aligned, stream);
   // One launch per group of slices, each writing its own columns of mid and
   // of the split sums (same values as one launch over all slices), then one
   // reduction over every column.
@@ -857,7 +868,7 @@ hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, bool aligne
     g.mid = static_cast<raw*>(args.mid) + static_cast<int64_t>(s0) * args.r_max;
     g.partials = args.partials ? args.partials + static_cast<int64_t>(s0) * args.r_max : nullptr;
     g.skip_reduce = 1;
-    const hipError_t e = aligned ? launch_al<T, true>(p, g, stream) : launch_al<T, false>(p, g, stream);
+    const hipError_t e = launch_group<T>(p, g, dtype, aligned, stream);
     if (e != hipSuccess) return e;
   }
   if (p.ks == 1 || args.skip_reduce) return hipSuccess;
@@ -866,8 +877,35 @@ hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, bool aligne
 
 }  // namespace
 
-bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, int num_cus,
-                 ShrinkPlan* plan) {
+// Whether the shrink runs as one launch of 16-row tiles over the whole
+// reduction (shrink_wide.hip) rather than split over workgroups.  A CU loads
+// such a tile's rows (x and every A block) at 60-85 GB/s, so what counts is
+// the bytes a CU loads, tile after tile.  Measured (whole calls, us, split vs
+// wide):
+//   16-bit, 4096 wide, rank 8 / 32 / 64 (256 / 384 / 640 KB a tile): 60 rows
+//     11.0 / 11.8 / 14.9 vs 10.2 / 11.6 / 15.6; 600 rows 13.8 / 14.5 / 18.2 vs
+//     12.3 / 13.7 / 19.8; 3900 rows 24.2 / 26.5 / 33.7 vs 21.7 / 24.1 / 31.1;
+//     1088 mixed rows to q|k|v at rank 16 (512 KB) 24.3 vs 24.7;
+//   unaligned 16-bit rows, which have no other staged form: K 4101, 4075 rows
+//     at rank 64 93.6 vs 40.6; K 14001, 958 rows at rank 64 (2.2 MB) 74.4 vs
+//     60.6; K 1001, 300 rows 27.0 vs 18.6;
+//   fp32: 958 rows at rank 16 (512 KB) 23.9 vs 21.1, rank 64 (1.3 MB) 43.5 vs
+//     44.9; 4075 rows, two slices at rank 64 (2.3 MB) 184.7 vs 129.1;
+//   decode-shaped calls (no segment over 16 rows: the split's expand adds the
+//     sums itself): fp32, 128 rows at rank 16 25.9 vs 22.6, 256 rows to q|k|v
+//     at rank 32 282 vs 104, but 8 rows 10.8 vs 13.8; K 4101, 64 rows 13.2 vs
+//     15.4.
+bool wide_pays(int in_dim, int launch_blocks, int blocks, int tiles, int max_len, int dtype, bool aligned, int num_cus) {
+  if (max_len <= 16 && tiles < num_cus / 2) return false;
+  const int64_t bytes = static_cast<int64_t>(launch_blocks + 1) * 16 * in_dim * (dtype == MLORA_F32 ? 4 : 2);
+  if (dtype == MLORA_F32) return bytes <= (1100 << 10) || tiles >= num_cus / 2;
+  if (!aligned) return true;
+  const int64_t rounds = (static_cast<int64_t>(tiles) + num_cus - 1) / num_cus;
+  return blocks == launch_blocks && bytes * rounds <= (400 << 10);
+}
+
+bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, bool aligned,
+                 int num_cus, ShrinkPlan* plan) {
   if (in_dim <= 0 || r_max <= 0 || n_slices < 1 || n_slices > kMaxSlices || bs < 0 || max_len < 0 || rows < 0)
     return false;
   const int kstep = (dtype == MLORA_F32) ? F32::KSTEP : BF16::KSTEP;
@@ -881,6 +919,17 @@ bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_
   p.nbt = 1;
   while (p.nbt < blocks) p.nbt *= 2;
   if (p.nbt > 16) return false;
+  const int tiles16 = static_cast<int>(std::min<int64_t>(
+      dense_tiles(bs, cdiv(max_len > 0 ? max_len : 1, 16), rows, 16), INT32_MAX));
+  if (p.nbt <= 8 && wide_pays(in_dim, blocks, n_slices * per_slice, tiles16, max_len, dtype, aligned, num_cus)) {
+    p.wide = 1;
+    p.bm = 16;
+    p.m_tiles = cdiv(max_len > 0 ? max_len : 1, p.bm);
+    p.ks = 1;
+    p.k_per_split = in_dim;
+    *plan = p;
+    return true;
+  }
   const int rb = 1;  // kShrinkRb
   p.bm = (max_len <= 16) ? 16 : 64 * rb;
   p.m_tiles = cdiv(max_len > 0 ? max_len : 1, p.bm);
@@ -946,22 +995,15 @@ bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_
 }
 
 hipError_t launch_shrink(const ShrinkPlan& plan, ShrinkArgs args, int dtype, bool aligned, hipStream_t stream) {
-  ShrinkPlan p = plan;
-  if (p.bm > 64 && !aligned) {
-    // 128-row tiles are the streamed kernel's, which needs aligned rows; the
-    // register-staged kernels take 64-row tiles, at most twice as many a
-    // segment.
-    p.bm = 64;
-    p.m_tiles *= 2;
-  }
+  const ShrinkPlan& p = plan;
   args.m_tiles = p.m_tiles;
   args.ks = p.ks;
   args.k_per_split = p.k_per_split;
   args.part_cols = args.n_slices * args.r_max;
   switch (dtype) {
-    case MLORA_BF16: return launch_dtype<BF16>(p, args, aligned, stream);
-    case MLORA_F16: return launch_dtype<F16>(p, args, aligned, stream);
-    default: return launch_dtype<F32>(p, args, aligned, stream);
+    case MLORA_BF16: return launch_dtype<BF16>(p, args, dtype, aligned, stream);
+    case MLORA_F16: return launch_dtype<F16>(p, args, dtype, aligned, stream);
+    default: return launch_dtype<F32>(p, args, dtype, aligned, stream);
   }
 }
 
