@@ -343,6 +343,31 @@ int mlora_pool_scatter(const void* stage, int64_t stage_row_stride, int32_t h, c
                        const mlora_pool_key* keys, int32_t n_keys, int32_t rank, int32_t num_slots,
                        int64_t max_numel, int32_t dtype, void* stream);
 
+/* Attention of one new token per sequence over a static KV cache, in one
+ * launch: q [batch, heads * D] and k [batch, kv_heads * D] are rotated
+ * (x * cos + roll(x, D / 2) * sin, cos and sin [batch or 1, D] of the data
+ * dtype, row stride rot_row_stride, 0 to share one row), k and v go into
+ * keys [batch, kv_heads, D, len] and values [batch, kv_heads, len, D] at
+ * position *pos (device memory, int64; outside [0, len) nothing is written),
+ * and out [batch, heads * D] = softmax(scale * q . keys, positions with a
+ * nonzero hide[batch or 1, len] byte left out) . values, fp32 math.
+ * Requirements (else -2): bf16 or fp16; D 64 or 128; heads / kv_heads 1, 2, 4
+ * or 8; len <= 2048; values 16-byte aligned.
+ * No counterpart is called in the reference (its model runs its own
+ * attention, multi_lora/graph_decode.py:23-111). */
+int mlora_decode_attention(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+                           int64_t v_row_stride, const void* cos, const void* sin, int64_t rot_row_stride, void* keys,
+                           void* values, const void* hide, int64_t hide_row_stride, const int64_t* pos, void* out,
+                           int64_t out_row_stride, int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                           int32_t len, float scale, int32_t dtype, void* stream);
+
+/* out[rows, width] = silu(gate) * up, fp32 math and one rounding; gate and up
+ * share a row stride, out is contiguous.  bf16 or fp16, width and strides
+ * multiples of 8, 16-byte aligned (else -2).  No counterpart is called in
+ * the reference. */
+int mlora_silu_mul(const void* gate, const void* up, int64_t in_row_stride, void* out, int32_t rows, int32_t width,
+                   int32_t dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -42,6 +42,8 @@ EXPORTS = (
     "mlora_build_plan",
     "mlora_apply_grouped_static",
     "mlora_rmsnorm_apply_grouped",
+    "mlora_decode_attention",
+    "mlora_silu_mul",
 )
 
 # include/mlora_hip.h: MLORA_STATIC_SCRATCH_BYTES
@@ -166,6 +168,12 @@ _SIGNATURES = {
         [_vp, _i64, _i32, _i32, ctypes.POINTER(Slice), _i32, _i32, _vp, _i64, ctypes.POINTER(SegMeta), _i32, _i32,
          _i32, _vp],
     ),
+    "mlora_decode_attention": (
+        ctypes.c_int,
+        [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32,
+         _i32, _f32, _i32, _vp],
+    ),
+    "mlora_silu_mul": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i32, _i32, _i32, _vp]),
     "mlora_build_plan": (ctypes.c_int, [ctypes.POINTER(SegMeta), _i32, _vp, _i32, _vp]),
     "mlora_rmsnorm_apply_grouped": (
         ctypes.c_int,

@@ -661,6 +661,55 @@ int mlora_add_rmsnorm(const void* x, int64_t x_row_stride, void* residual, int64
                       rows, hidden, eps, dtype, stream);
 }
 
+int mlora_decode_attention(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+                           int64_t v_row_stride, const void* cos, const void* sin, int64_t rot_row_stride, void* keys,
+                           void* values, const void* hide, int64_t hide_row_stride, const int64_t* pos, void* out,
+                           int64_t out_row_stride, int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                           int32_t len, float scale, int32_t dtype, void* stream) {
+  g_err[0] = '\0';
+  if (dtype != MLORA_BF16 && dtype != MLORA_F16) return fail(kUnsupported, "decode attention needs bf16 or fp16, got dtype %d", dtype);
+  if (batch < 0 || heads < 1 || kv_heads < 1 || len < 1 || heads % kv_heads != 0)
+    return fail(kBadArg, "batch %d, heads %d, kv_heads %d, len %d", batch, heads, kv_heads, len);
+  const int rep = heads / kv_heads;
+  if ((head_dim != 64 && head_dim != 128) || (rep != 1 && rep != 2 && rep != 4 && rep != 8) || len > mlora::kAttnMaxLen ||
+      !al16(values) || static_cast<int64_t>(batch) * kv_heads > mlora::kMaxBlocks)
+    return fail(kUnsupported, "decode attention takes head_dim 64 or 128 (got %d), 1, 2, 4 or 8 heads a key head (%d), "
+                "caches of up to %d (%d), 16-byte aligned values", head_dim, rep, mlora::kAttnMaxLen, len);
+  if (batch == 0) return 0;
+  if (!q || !k || !v || !cos || !sin || !keys || !values || !hide || !pos || !out) return fail(kBadArg, "null pointer");
+  const int64_t qw = static_cast<int64_t>(heads) * head_dim, kw = static_cast<int64_t>(kv_heads) * head_dim;
+  if (q_row_stride < qw || k_row_stride < kw || v_row_stride < kw || out_row_stride < qw || rot_row_stride < 0 ||
+      hide_row_stride < 0)
+    return fail(kBadArg, "row strides do not hold the rows");
+  mlora::AttnArgs a{};
+  a.q = q, a.k = k, a.v = v;
+  a.q_stride = q_row_stride, a.k_stride = k_row_stride, a.v_stride = v_row_stride;
+  a.cos = cos, a.sin = sin, a.rot_stride = rot_row_stride;
+  a.keys = keys, a.values = values;
+  a.hide = static_cast<const uint8_t*>(hide), a.hide_stride = hide_row_stride;
+  a.pos = pos;
+  a.out = out, a.out_stride = out_row_stride;
+  a.batch = batch, a.kv_heads = kv_heads, a.len = len;
+  a.scale = scale;
+  const hipError_t e = mlora::launch_decode_attn(a, dtype, head_dim, rep, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "decode attention launch");
+  return 0;
+}
+
+int mlora_silu_mul(const void* gate, const void* up, int64_t in_row_stride, void* out, int32_t rows, int32_t width,
+                   int32_t dtype, void* stream) {
+  g_err[0] = '\0';
+  if (dtype != MLORA_BF16 && dtype != MLORA_F16) return fail(kUnsupported, "silu_mul needs bf16 or fp16, got dtype %d", dtype);
+  if (rows < 0 || width < 1 || in_row_stride < width) return fail(kBadArg, "rows %d, width %d, row stride %lld", rows, width, (long long)in_row_stride);
+  if (rows == 0) return 0;
+  if (gate == nullptr || up == nullptr || out == nullptr) return fail(kBadArg, "null pointer");
+  if (width % 8 != 0 || in_row_stride % 8 != 0 || !al16(gate) || !al16(up) || !al16(out))
+    return fail(kUnsupported, "silu_mul needs 16-byte aligned rows");
+  const hipError_t e = mlora::launch_silu_mul(gate, up, in_row_stride, out, rows, width, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "silu_mul launch");
+  return 0;
+}
+
 int mlora_pool_scatter(const void* stage, int64_t stage_row_stride, int32_t h, const int32_t* slots,
                        const mlora_pool_key* keys, int32_t n_keys, int32_t rank, int32_t num_slots,
                        int64_t max_numel, int32_t dtype, void* stream) {

@@ -312,6 +312,28 @@ struct ScatterArgs {
 
 hipError_t launch_scatter(const ScatterArgs& args, int64_t max_numel, int elem_bytes, hipStream_t stream);
 
+// -------------------------------------------------------------- decoder
+// Longest cache the decode attention's scores fit in LDS for.
+constexpr int kAttnMaxLen = 2048;
+
+struct AttnArgs {
+  const void *q, *k, *v;  // rows of the new tokens [batch, heads * D]
+  int64_t q_stride, k_stride, v_stride;
+  const void *cos, *sin;  // [batch or 1, D]
+  int64_t rot_stride;
+  void *keys, *values;    // [batch, kv_heads, D, len] and [batch, kv_heads, len, D]
+  const uint8_t* hide;    // [batch or 1, len]: nonzero = not attended
+  int64_t hide_stride;
+  const int64_t* pos;     // the new token's cache position (device)
+  void* out;              // [batch, heads * D]
+  int64_t out_stride;
+  int batch, kv_heads, len;
+  float scale;
+};
+hipError_t launch_decode_attn(const AttnArgs& args, int dtype, int head_dim, int rep, hipStream_t stream);
+hipError_t launch_silu_mul(const void* gate, const void* up, int64_t in_stride, void* out, int rows, int width, int dtype,
+                           hipStream_t stream);
+
 // Base pointer of slice `s`'s A (or B) for one slot, selected with
 // compile-time indexing so the kernel-argument array is never indexed
 // dynamically.

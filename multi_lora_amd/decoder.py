@@ -16,7 +16,9 @@ contiguous operands, the score scale applied inside the first) with the
 softmax in fp32; the query heads that share a key head are stacked as rows,
 so keys are never repeated.  Rotary runs once per layer over q and k
 together when they are adjacent columns of one projection output (the fused
-q|k|v group's).  A block's residual adds travel to the next RMSNorm, which
+q|k|v group's).  On the GPU, a decode step's rotary, cache write and
+attention are one HIP launch, and so is the MLP's SiLU gate
+(``kernels/decode_attn.py``; 16-bit data).  A block's residual adds travel to the next RMSNorm, which
 ``fuse_rmsnorm`` turns into one fused add + RMSNorm kernel.  The KV cache is
 written in place at ``cache_position`` and read whole under a boolean mask,
 so a decode step touches fixed addresses and can be captured in a HIP graph.
@@ -35,6 +37,8 @@ from typing import List, Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+
+from .kernels.decode_attn import decode_attention, silu_mul
 
 
 @dataclass
@@ -148,8 +152,16 @@ class Attention(nn.Module):
 
     def forward(self, x, rot: Rotary, hide, kv: Optional[StaticKV], layer: int, cache_position):
         b, t, _ = x.shape
-        q, k = self._rotate_qk(self.q_proj(x).reshape(b * t, -1), self.k_proj(x).reshape(b * t, -1), rot)
-        out = self._attend(q, k, self.v_proj(x), b, t, hide, kv, layer, cache_position)
+        q, k = self.q_proj(x).reshape(b * t, -1), self.k_proj(x).reshape(b * t, -1)
+        v = self.v_proj(x)
+        if t == 1 and kv is not None and q.is_cuda:
+            # One new token a sequence: rotary, cache and attention in one launch.
+            out = decode_attention(q, k, v.reshape(b, -1), rot.cos, rot.sin, kv.keys[layer], kv.values[layer], hide,
+                                   cache_position, self.scale)
+            if out is not None:
+                return self.o_proj(out.view(b, 1, -1))
+        q, k = self._rotate_qk(q, k, rot)
+        out = self._attend(q, k, v, b, t, hide, kv, layer, cache_position)
         return self.o_proj(out.to(x.dtype))
 
     def _rotate_qk(self, q: torch.Tensor, k: torch.Tensor, rot: Rotary):
@@ -229,7 +241,9 @@ class MLP(nn.Module):
         self.down_proj = nn.Linear(c.intermediate_size, c.hidden_size, bias=False)
 
     def forward(self, x):
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        gate, up = self.gate_proj(x), self.up_proj(x)
+        act = silu_mul(gate, up) if gate.is_cuda else None
+        return self.down_proj(F.silu(gate) * up if act is None else act)
 
 
 class Block(nn.Module):
