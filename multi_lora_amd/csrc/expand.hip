@@ -45,13 +45,13 @@ __global__ __launch_bounds__(256) void expand_kernel(ExpandArgs a) {
 // Streamed form for long segments (16-bit types, aligned rows, 64-row tiles,
 // four workgroups a CU); the body is expand_dma_tile (NT: non-temporal
 // output tile).
-template <class T, int BM, bool NT>
+template <class T, int BM, bool NT, int CB>
 __global__ __launch_bounds__(256, 4) void expand_dma_kernel(ExpandArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char tile[expand_dma_lds_bytes<BM>()];
+  __shared__ __attribute__((aligned(1024))) unsigned char tile[expand_dma_lds_bytes<BM, CB>()];
   const int bid = blockIdx.x;
   TileRef tr;
   if (!dense_tile(a.meta, a.rows, bid / a.n_tiles, BM, &tr)) return;
-  expand_dma_tile<T, BM, NT>(a, tr, bid % a.n_tiles, tile);
+  expand_dma_tile<T, BM, NT, CB>(a, tr, bid % a.n_tiles, tile);
 }
 
 template <class T, int BM, bool AL>
@@ -77,6 +77,20 @@ hipError_t launch_al(const ExpandArgs& args, bool aligned, hipStream_t stream) {
 
 }  // namespace
 
+// Row-order loads for r_max 17 to 64 (expand_dma.h).  At 16 and below a
+// fragment load's four neighbouring lanes lie in one cache line already; past
+// 64 the side area would cost a workgroup a CU.
+template <class T, bool NT>
+void launch_streamed_cb(const ExpandArgs& args, unsigned blocks, hipStream_t stream) {
+  constexpr int BM = kExpandStreamBM;
+  if (args.r_max > 64 || args.r_max <= 16)
+    hipLaunchKernelGGL((expand_dma_kernel<T, BM, NT, 0>), dim3(blocks), dim3(256), 0, stream, args);
+  else if (args.r_max > 32)
+    hipLaunchKernelGGL((expand_dma_kernel<T, BM, NT, 8>), dim3(blocks), dim3(256), 0, stream, args);
+  else
+    hipLaunchKernelGGL((expand_dma_kernel<T, BM, NT, 4>), dim3(blocks), dim3(256), 0, stream, args);
+}
+
 template <class T>
 hipError_t launch_streamed(ExpandArgs args, hipStream_t stream) {
   constexpr int BM = kExpandStreamBM;
@@ -92,11 +106,9 @@ hipError_t launch_streamed(ExpandArgs args, hipStream_t stream) {
   // launch of about one round the hint costs: prefill down (1104 tiles)
   // 17.3 -> 20.1 us.
   if (args.cus > 0 && blocks >= static_cast<int64_t>(kStreamNtTilesPerCu) * args.cus)
-    hipLaunchKernelGGL((expand_dma_kernel<T, BM, true>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
-                       args);
+    launch_streamed_cb<T, true>(args, static_cast<unsigned>(blocks), stream);
   else
-    hipLaunchKernelGGL((expand_dma_kernel<T, BM, false>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
-                       args);
+    launch_streamed_cb<T, false>(args, static_cast<unsigned>(blocks), stream);
   return hipGetLastError();
 }
 

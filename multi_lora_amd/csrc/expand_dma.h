@@ -15,8 +15,9 @@ typedef __attribute__((address_space(3))) void lvoid_t;
 
 // Bytes of LDS the tile needs (BM rows of 256 columns, 16-bit), to be
 // aligned to 1024 bytes.
-template <int BM>
-constexpr int expand_dma_lds_bytes() { return BM * kExpandBN * 2; }
+// CB > 0: and a side area, BM rows of CB chunks (64 rows: 8 or 4 KB).
+template <int BM, int CB = 0>
+constexpr int expand_dma_lds_bytes() { return BM * kExpandBN * 2 + BM * CB * 16; }
 
 // Tile `tr` (rows [tr.start + tr.mt * BM, ...) of one segment), column tile
 // nt_g of the call's slices; `tile` is expand_dma_lds_bytes<BM>() of LDS.
@@ -31,7 +32,18 @@ constexpr int expand_dma_lds_bytes() { return BM * kExpandBN * 2; }
 // chunk p ^ (r & 15), which spreads both the MFMA-layout accesses (16 rows,
 // one chunk each) and the row reads over the banks.  The rounded delta is
 // added into the tile in place, then whole rows are stored.
-template <class T, int BM, bool NT = false>
+//
+// CB (8 or 4; r_max up to 64 or 32): B and mid are loaded in row order, CB
+// neighbouring lanes to a row's chunks, all of them before the tile, and the
+// fragments are formed through the side area: B's 16 columns at a time in the
+// wave's own part, then the workgroup's mid rows once for all four waves.
+// CB 0 loads fragments directly: from rows wider than 32 bytes every four
+// neighbouring lanes then ask for two to four cache lines (decode.hip,
+// shrink_chunk), every wave loads the same mid rows, and a second K-step's
+// loads wait behind the tile's.  Prefill gate|up (4075 rows, ranks 16, 32 and
+// 64 in r_max 64): the call 117.2 -> 104.9 us, its expand about 85 us for 467
+// MB of output read and written (5.5 TB/s); down 47.2 -> 45.5.
+template <class T, int BM, bool NT = false, int CB = 0>
 __device__ __forceinline__ void expand_dma_tile(const ExpandArgs& a, const TileRef& tr, int nt_g,
                                                 unsigned char* tile) {
   using raw = typename T::raw_t;
@@ -67,14 +79,16 @@ __device__ __forceinline__ void expand_dma_tile(const ExpandArgs& a, const TileR
   const raw* B = static_cast<const raw*>(a.slices[s].b) + static_cast<int64_t>(pslot) * a.slices[s].b_slot_stride;
   const int64_t brs = a.slices[s].b_row_stride;
   const raw* brow[4];
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb)
-    brow[nb] = B + static_cast<int64_t>(min(n0 + (wave * 4 + nb) * 16 + r16, out_dim - 1)) * brs;
   const raw* mrow[TB];
+  if constexpr (CB == 0) {
 #pragma unroll
-  for (int tb = 0; tb < TB; ++tb)
-    mrow[tb] = static_cast<const raw*>(a.mid) + s * a.r_max +
-               static_cast<int64_t>(min(row0 + tb * 16 + r16, end - 1)) * a.mid_stride;
+    for (int nb = 0; nb < 4; ++nb)
+      brow[nb] = B + static_cast<int64_t>(min(n0 + (wave * 4 + nb) * 16 + r16, out_dim - 1)) * brs;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+      mrow[tb] = static_cast<const raw*>(a.mid) + s * a.r_max +
+                 static_cast<int64_t>(min(row0 + tb * 16 + r16, end - 1)) * a.mid_stride;
+  }
 
   // The slot's rank and scaling word go out first, as vector loads (lane0 is
   // 0 in every lane, but not known to be uniform), and are waited for
@@ -92,7 +106,21 @@ __device__ __forceinline__ void expand_dma_tile(const ExpandArgs& a, const TileR
   // unmasked (masked at the MFMA): loads complete in issue order, so waiting
   // for them leaves the tile's loads in flight.
   u32x4 yv0[TB], bv0[4];
-  {
+  constexpr int LPB = CB > 0 ? CB : 8;       // lanes a row
+  constexpr int BROWS = 64 / LPB;            // B rows an instruction
+  constexpr int BI = 64 / BROWS;             // instructions for the wave's 64 columns
+  constexpr int YI = (BM * LPB + 255) / 256; // mid chunks a thread
+  u32x4 braw[CB > 0 ? BI : 1], yraw[CB > 0 ? YI : 1];
+  if constexpr (CB > 0) {
+    const int kk = (tid % LPB) * VEC < a.r_max ? (tid % LPB) * VEC : 0;
+#pragma unroll
+    for (int i = 0; i < YI; ++i)
+      yraw[i] = ld_chunk(static_cast<const raw*>(a.mid) + s * a.r_max + kk +
+                         static_cast<int64_t>(min(row0 + (tid + i * 256) / LPB, end - 1)) * a.mid_stride);
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+      braw[i] = ld_chunk(B + static_cast<int64_t>(min(n0 + wave * 64 + i * BROWS + lane / LPB, out_dim - 1)) * brs + kk);
+  } else {
     const int kk = g * VEC;
     const int off = kk < a.r_max ? kk : 0;
 #pragma unroll
@@ -138,14 +166,59 @@ __device__ __forceinline__ void expand_dma_tile(const ExpandArgs& a, const TileR
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  {
+  if constexpr (CB > 0) {
+    constexpr int RS = CB / 4;           // K-steps
+    constexpr int ROW = CB * 16;         // bytes of a side row
+    unsigned char* side = tile + BM * ROWB;
+    // Chunk c of side row r sits at c ^ swz(r): a fragment read's 16 rows fall
+    // on 16 different 16-byte bank groups.
+    auto swz = [](int r) { return CB == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
+    auto put = [&](unsigned char* area, int r, const u32x4& v) {
+      *reinterpret_cast<u32x4*>(area + r * ROW + (((tid % LPB) ^ swz(r)) << 4)) = v;
+    };
+    auto frag = [&](const unsigned char* area, int r, int ks) {
+      return *reinterpret_cast<const u32x4*>(area + r * ROW + (((ks * 4 + g) ^ swz(r)) << 4));
+    };
+    u32x4 bf[RS][4];
+    unsigned char* mine = side + wave * 16 * ROW;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+#pragma unroll
+      for (int i = 0; i < 16 / BROWS; ++i) put(mine, i * BROWS + lane / LPB, braw[nb * (16 / BROWS) + i]);
+#pragma unroll
+      for (int ks = 0; ks < RS; ++ks) bf[ks][nb] = frag(mine, r16, ks) & keep_mask<T>(rank - ks * KSTEP - g * VEC);
+    }
+    // Barriers that wait for this wave's LDS accesses only: a fence on the
+    // LDS would also wait for the tile, which is on its way there.
+    auto side_barrier = [] {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    side_barrier();
+#pragma unroll
+    for (int i = 0; i < YI; ++i) put(side, (tid + i * 256) / LPB, yraw[i]);
+    side_barrier();
+#pragma unroll
+    for (int ks = 0; ks < RS; ++ks) {
+      if (ks * KSTEP >= rank) break;
+      const u32x4 m = keep_mask<T>(rank - ks * KSTEP - g * VEC);
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        const u32x4 yv = frag(side, tb * 16 + r16, ks) & m;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[nb][tb] = T::mma(acc[nb][tb], bf[ks][nb], yv);
+      }
+    }
+  } else {
     const u32x4 m = keep_mask<T>(rank - g * VEC);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = T::mma(acc[nb][tb], bv0[nb] & m, yv0[tb] & m);
   }
-  for (int k0 = KSTEP; k0 < rank; k0 += KSTEP) {
+  for (int k0 = KSTEP; CB == 0 && k0 < rank; k0 += KSTEP) {
     const int kk = k0 + g * VEC;
     const int valid = rank - kk;
     u32x4 yv[TB];

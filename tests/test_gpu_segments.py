@@ -411,3 +411,19 @@ def test_mixed_batch_expand_in_a_replayed_graph_follows_table_rewrites(dev):
                        cols, workspace=Workspace())
         torch.cuda.synchronize()
         assert torch.equal(out.cpu(), want.cpu()), f"replay {rep}"
+
+
+@pytest.mark.parametrize("r_max,ranks", [(16, [16, 9]), (24, [24, 7]), (32, [32, 17]), (40, [40, 33]), (64, [64, 20]),
+                                         (72, [72, 30])])
+def test_streamed_expand_forms(dev, r_max, ranks):
+    """Long segments over outputs wide enough for the streamed 64-row tiles:
+    fragments loaded directly (r_max 16, 72) and through the side area with
+    rows of four (24, 32) and eight chunks (40, 64), with a ragged last column
+    tile and row tile and a rank-0 segment."""
+    lens, slots, ranks = [1030, 70, 129], [0, 2, 1], ranks + [0]
+    x, As, Bs, base, cols, meta_cpu, scal = case(dev, lens, slots, ranks, 64, [13000, 264], r_max, torch.bfloat16, r_max)
+    got = base.to(dev)
+    apply_segments(x.to(dev), [a.to(dev) for a in As], [b.to(dev) for b in Bs],
+                   make_meta(lens, slots, ranks, scal, dev, torch.bfloat16), got, cols, workspace=Workspace())
+    assert_tol_f64(got.cpu(), apply_f64(x, As, Bs, meta_cpu, base, cols), f"r_max {r_max}")
+    assert torch.equal(got[1030:1100].cpu(), base[1030:1100])
