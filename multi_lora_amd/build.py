@@ -91,7 +91,11 @@ def _build_calls(_=None) -> None:
     root = Path(torch.__file__).resolve().parent
     rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
     tmp = CALLS_MODULE.with_suffix(".so.tmp")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    # NDEBUG as torch itself is built: without it pybind11's reference counting
+    # (in torch's headers) gives the module a thread-local block that nothing
+    # touches, and glibc then looks every thread-local access of the process up
+    # the slow way (torch's own calls from Python 20 % slower, 0.9 us an upload).
+    cmd = ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            *(f"-isystem{d}" for d in (root / "include", root / "include/torch/csrc/api/include", rocm / "include",
                                       sysconfig.get_paths()["include"])),
