@@ -997,15 +997,21 @@ hipError_t launch_norm_shrink(const int32_t* plan, const DecodeArgs& a, const No
   const int64_t grid_y = n_norm + (a.item_fast ? a.e_grid : n_shrink);
   if (grid_y > 65535 || !grid_fits(grid_y * per_row)) return hipErrorInvalidConfiguration;
   const dim3 grid(static_cast<unsigned>(per_row), static_cast<unsigned>(grid_y));
-  // A grid of at most four workgroups a CU runs at once and is bound by one
-  // workgroup's latency: direct loads (a layer of 14 rows over one adapter:
-  // 37.5 against 38.2 us).
-  if (!a.item_fast)
-    hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kDirect>), grid, dim3(256), 0, stream, plan, a.plan_cap,
-                       static_cast<int>(n_norm), a, na);
-  else
-    hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kStaged>), grid, dim3(256), 0, stream, plan, a.plan_cap,
-                       static_cast<int>(n_norm), a, na);
+  // Direct loads for a grid of at most four workgroups a CU, which runs at once
+  // and is bound by one workgroup's latency (a layer of 14 rows over one
+  // adapter: 37.5 against 38.2 us), and for items of one or two A blocks: the
+  // norm rows share the launch, and the LDS that staging takes (24 KB a
+  // workgroup) keeps waves off the CU that direct loads let run (q|k|v of 256
+  // rows, 112 rank-32 adapters, the whole call: 39.1 against 40.7 us staged).
+  if constexpr (NBT > 2) {
+    if (a.item_fast) {
+      hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kStaged>), grid, dim3(256), 0, stream, plan,
+                         a.plan_cap, static_cast<int>(n_norm), a, na);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kDirect>), grid, dim3(256), 0, stream, plan, a.plan_cap,
+                     static_cast<int>(n_norm), a, na);
   return hipGetLastError();
 }
 
