@@ -229,14 +229,14 @@ def calls():
     handle = lib()
     with _lock:
         if _calls_module is None:
-            from .batch_info import PLAN_LONG_ROWS, KernelInputMetaData
+            from .batch_info import KernelInputMetaData
             try:
                 from . import _calls as module
             except ImportError as e:
                 raise RuntimeError(f"{LIB_PATH.parent / '_calls.so'} is not built ({e}); run "
                                    "`python -m multi_lora_amd.build`") from e
             module.set_library(tuple(ctypes.cast(getattr(handle, f), ctypes.c_void_p).value for f in _CALLS_FUNCTIONS),
-                               MloraError, KernelInputMetaData, PLAN_LONG_ROWS)
+                               MloraError, KernelInputMetaData)
             _calls_module = module
     return _calls_module
 

@@ -18,7 +18,7 @@ import torch
 
 from .. import _ffi
 from ..kernels.lora_ops import (GROUPED_MAX_LEN, LinkedWorkspace, Workspace, apply_grouped, apply_segments, expand,
-                                 planned_pays, reserve_segments, rmsnorm_apply_grouped, shrink)
+                                 rmsnorm_apply_grouped, shrink)
 from ..kernels.rmsnorm import rmsnorm_fwd
 from .base import LoRABackend
 
@@ -59,8 +59,7 @@ class HipLoRABackend(LoRABackend):
         """Add each segment's LoRA delta into ``base_output`` (in place) and return it.
 
         Decode-shaped batches (every segment at most 16 rows) take the
-        slot-grouped path, which reads each referenced adapter once per call,
-        and so do batches with a few hundred prompt rows (``planned_pays``);
+        slot-grouped path, which reads each referenced adapter once per call;
         other batches run the segment shrink and expand in one library call.
         """
         return self.apply_lora_multi(x, [a_stack], [b_stack], base_output, [0])
@@ -95,11 +94,9 @@ class HipLoRABackend(LoRABackend):
         x = x.contiguous()
         a_stacks = [a.contiguous() for a in a_stacks]
         b_stacks = [b.contiguous() for b in b_stacks]
-        if (meta.max_len <= GROUPED_MAX_LEN or planned_pays(meta, x, a_stacks, b_stacks)) and apply_grouped(
+        if meta.max_len <= GROUPED_MAX_LEN and apply_grouped(
             x, a_stacks, b_stacks, meta, base_output, col_offsets, workspace=self.linked_workspace,
         ):
-            if meta.max_len > GROUPED_MAX_LEN:
-                reserve_segments(x, a_stacks, meta, self.workspace)
             return base_output
         return apply_segments(x, a_stacks, b_stacks, meta, base_output, col_offsets, workspace=self.workspace)
 

@@ -34,11 +34,6 @@ PLAN_HEADER_WORDS = 16
 PLAN_ENTRY_WORDS = 32
 PLAN_ROWS = 16
 PLAN_ROW_WORD = 8
-# Tables of segments of more than 16 rows get room for their whole plan up to
-# this many rows; longer ones run faster as segments (4096 -> 4096 at rank 16,
-# 1600 rows: 18.1 us planned, 17.5 as segments) and would only make the
-# table's copy longer.
-PLAN_LONG_ROWS = 1600
 
 
 def plan_words(cap: int) -> int:
@@ -160,25 +155,6 @@ class KernelInputMetaData:
             got = self._summaries[num_slots] = (len(long_lens), sum(long_lens), len(short))
         return got
 
-    def plan_is_current(self, rows: int) -> bool:
-        """Whether the plan describes the table as it stands, for a call of ``rows`` rows.
-
-        A table of segments of at most 16 rows is only ever applied through
-        its plan.  Longer ones were first applied from the columns, so their
-        plan counts only while nothing but ``write_kernel_input_metadata``
-        has touched the packed columns (torch bumps the buffer's version on
-        every in-place write), every entry fits, and no planned row lies past
-        the call's rows (workspace positions count planned rows)."""
-        pk = self.packed
-        if pk is None or self.plan is None:
-            return False
-        c = pk.dev_cols
-        return (self.plan is c["plan"] and self.weight_indices is c["weight_indices"]
-                and self.seg_indptr is c["seg_indptr"] and self.lora_ranks is c["lora_ranks"]
-                and self.scalings is c["scalings"] and self.bs == pk.written_bs and self.plan_cap == pk.plan_cap
-                and self.plan_entries == pk.plan_entries and pk.dev._version == pk.written_version
-                and 0 < pk.plan_entries <= pk.plan_cap and pk.written_rows <= rows)
-
     def set_host_copies(self, lens: Sequence[int], slots: Sequence[int]) -> None:
         self.host_lens = list(lens)
         self.host_slots = list(slots)
@@ -191,19 +167,16 @@ class PackedColumns:
     Layout (each section 64-byte aligned): weight_indices[capacity],
     seg_lens[capacity], seg_indptr[capacity + 1] (int32), lora_ranks[num_slots]
     (int32), scalings[num_slots] (the pool dtype), then the plan (int32, room
-    for capacity + min(capacity, num_slots) entries, so that every table of
-    segments of at most 16 rows fits, and for every table of at most ``rows``
-    rows in all).  ``write`` fills the mirror, builds the plan in
+    for capacity + min(capacity, num_slots) entries: every table of segments
+    of at most 16 rows fits).  ``write`` fills the mirror, builds the plan in
     it, and copies everything up to the plan's last entry in one transfer on
     the current stream; before touching the mirror it waits for the previous
     transfer to have read it.
     """
 
-    def __init__(self, capacity: int, num_slots: int, device: torch.device, dtype: torch.dtype, rows: int = 0) -> None:
+    def __init__(self, capacity: int, num_slots: int, device: torch.device, dtype: torch.dtype) -> None:
         self.capacity, self.num_slots = capacity, num_slots
-        # A slot's rows fill ceil(n / 16) entries: at most rows / 16 + one a
-        # segment (or a slot) in all.
-        self.plan_cap = max(1, max(capacity, -(-rows // PLAN_ROWS)) + min(capacity, num_slots))
+        self.plan_cap = max(1, capacity + min(capacity, num_slots))
         layout = [("weight_indices", capacity, torch.int32), ("seg_lens", capacity, torch.int32),
                   ("seg_indptr", capacity + 1, torch.int32), ("lora_ranks", num_slots, torch.int32),
                   ("scalings", num_slots, dtype), ("plan", plan_words(self.plan_cap), torch.int32)]
@@ -212,23 +185,17 @@ class PackedColumns:
             cur = (cur + 63) // 64 * 64
             offs.append((name, cur, n, dt))
             cur += n * torch.empty(0, dtype=dt).element_size()
-        # Made outside inference mode, so torch counts the writes to it
-        # (plan_is_current): an inference tensor has no version.
-        self.dev_cols: Dict[str, torch.Tensor] = {}
-        with torch.inference_mode(False):
-            self.dev = torch.zeros(max(cur, 1), dtype=torch.uint8, device=device)
-            for name, off, n, dt in offs:
-                self.dev_cols[name] = self.dev[off:off + n * dt.itemsize].view(dt)
+        self.dev = torch.zeros(max(cur, 1), dtype=torch.uint8, device=device)
         self.host = torch.zeros(max(cur, 1), dtype=torch.uint8, pin_memory=True)
+        self.dev_cols: Dict[str, torch.Tensor] = {}
         self.host_cols: Dict[str, torch.Tensor] = {}
         host_np = self.host.numpy()
         self.host_np = {}
         self.plan_off = offs[-1][1]
         self.plan_entries = 0
-        self.written_bs = self.written_rows = 0
-        self.written_version = -1
         for name, off, n, dt in offs:
             es = torch.empty(0, dtype=dt).element_size()
+            self.dev_cols[name] = self.dev[off:off + n * es].view(dt)
             self.host_cols[name] = self.host[off:off + n * es].view(dt)
             if dt == torch.int32:
                 self.host_np[name] = host_np[off:off + n * es].view(np.int32)
@@ -257,7 +224,6 @@ class PackedColumns:
             self.host_cols["scalings"].float().numpy(), self.num_slots, rows, np_cols["plan"])
         used = self.plan_off + 4 * plan_words(min(self.plan_entries, self.plan_cap))
         self.dev[:used].copy_(self.host[:used], non_blocking=True)
-        self.written_bs, self.written_rows, self.written_version = nb, rows, self.dev._version
         self.event.record()
         self.pending = True
 
@@ -377,7 +343,7 @@ def write_kernel_input_metadata(
 
     if rows > meta.weight_indices.shape[0] or meta.packed is not None:
         if device.type == "cuda":
-            pk = PackedColumns(rows, slots, device, dtype, rows=indptr[-1] if indptr[-1] <= PLAN_LONG_ROWS else 0)
+            pk = PackedColumns(rows, slots, device, dtype)
             pk.write(columns)
             c = pk.dev_cols
             fresh = KernelInputMetaData(bs=rows, seg_lens=c["seg_lens"], seg_indptr=c["seg_indptr"],

@@ -44,8 +44,7 @@ PyObject* launch_error = nullptr;  // exception type of a failed launch
 PyObject* meta_type = nullptr;     // KernelInputMetaData
 
 PyObject *s_bs, *s_max_len, *s_seg_indptr, *s_weight_indices, *s_lora_ranks, *s_scalings, *s_plan, *s_plan_cap,
-    *s_plan_entries, *s_table_summary, *s_plan_is_current, *s_bufs, *s_buf, *s_cuda, *s_get,
-    *s_device;
+    *s_plan_entries, *s_table_summary, *s_bufs, *s_buf, *s_cuda, *s_get, *s_device;
 
 constexpr int kUnsupported = -2;  // the library's "shape not eligible"
 
@@ -173,13 +172,6 @@ struct Table {
     }
     return true;
   }
-
-  bool plan_is_current(int64_t rows) {
-    Ref n(PyLong_FromLongLong(rows));
-    Ref r(PyObject_CallMethodObjArgs(meta, s_plan_is_current, n.p, nullptr));
-    if (r.p == nullptr) PyErr_Clear();
-    return r.p == Py_True;
-  }
 };
 
 hipStream_t stream_of(at::Device dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
@@ -294,36 +286,10 @@ struct Slices {
     }
     return true;
   }
-
-  // 256-column tiles of the output.
-  int64_t tiles() const {
-    int64_t c = 0;
-    for (int i = 0; i < n; ++i) c += (s[i].out_dim + 255) / 256;
-    return c;
-  }
 };
 
-// Whether a batch with segments of more than 16 rows takes the planned path
-// (kernels/lora_ops.py: planned_pays says why the line lies there).
-constexpr int64_t kPlannedLongBytes = 56 << 20;
-int64_t plan_long_rows = 0;  // batch_info.PLAN_LONG_ROWS
-
-bool planned_pays(Table& t, int64_t rows, int64_t in_dim, int64_t r_max, int n, int64_t tiles, hipStream_t stream) {
-  if (rows > plan_long_rows || t.m.plan == nullptr || t.m.plan_entries <= 0) return false;
-  const int64_t groups = n * r_max <= 64 ? 1 : n;
-  const int64_t cost = (in_dim + 255) / 256 * (16 * groups + n * r_max) + tiles * (r_max + 32);
-  if (t.m.plan_entries * cost * 512 > kPlannedLongBytes) return false;
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  if (capturing != hipStreamCaptureStatusNone) return false;
-  return t.plan_is_current(rows);
-}
-
-// HipLoRABackend.apply_lora_multi: planned path for decode-shaped batches and
-// small prompt batches, else segments.
+// HipLoRABackend.apply_lora_multi: planned path for decode-shaped batches,
+// else segments.
 Took apply_multi(PyObject* const* args) {
   PyObject *px = args[0], *pa = args[1], *pb = args[2], *pmeta = args[3], *pout = args[4], *pcols = args[5],
            *plinked = args[6], *pseg = args[7];
@@ -342,24 +308,14 @@ Took apply_multi(PyObject* const* args) {
   const int r_max = static_cast<int>(sl.r_max);
   const hipStream_t stream = stream_of(dev);
 
-  bool planned = t.m.max_len <= MLORA_PLAN_ROWS;  // decode-shaped
-  if (planned && t.m.plan == nullptr) return Took::kNo;  // the caller has one built
-  const bool long_planned = !planned && planned_pays(t, rows, in_dim, r_max, sl.n, sl.tiles(), stream);
-  planned = planned || long_planned;
   void* ws;
   size_t ws_bytes;
-  if (planned) {
+  if (t.m.max_len <= MLORA_PLAN_ROWS) {  // decode-shaped
+    if (t.m.plan == nullptr) return Took::kNo;  // the caller has one built
     const size_t need = lib.grouped_ws(in_dim, r_max, sl.n, rows, t.m.num_slots, dt, 0);
     if (need != 0) {
-      Took got = linked_workspace(plinked, need, *x, px, stream, &ws, &ws_bytes);
+      const Took got = linked_workspace(plinked, need, *x, px, stream, &ws, &ws_bytes);
       if (got != Took::kYes) return got;
-      // A prompt batch's segment workspace is kept at hand too (reserve_segments).
-      void* seg;
-      size_t seg_bytes;
-      if (long_planned) {
-        got = workspace(pseg, lib.segments_ws(in_dim, r_max, sl.n, rows, t.m.bs, t.m.max_len, dt), *x, px, &seg, &seg_bytes);
-        if (got != Took::kYes) return got;
-      }
       const int rc = unlocked([&] {
         return lib.grouped(x->data_ptr(), x->stride(0), rows, in_dim, sl.s, sl.n, r_max, out->data_ptr(), out->stride(0),
                            &t.m, dt, ws, ws_bytes, 0, 3, stream);
@@ -580,25 +536,10 @@ PyObject* py_add_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&](Took* took) { return norm(args[0], args[1], args[2], args[3], took); });
 }
 
-// planned_pays(meta, x, a_stacks, b_stacks) -> bool
-PyObject* py_planned_pays(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (!arity(n, 4)) return nullptr;
-  return guarded([&](Took*) -> PyObject* {
-    const at::Tensor* x = tensor_of(args[1]);
-    Slices sl;
-    Table t;
-    if (x == nullptr || !x->is_cuda() || !is_rows(*x) || !sl.read(args[2], args[3], Py_None, *x) ||
-        !t.read(args[0], x->device(), sl.slots))
-      Py_RETURN_FALSE;
-    return PyBool_FromLong(
-        planned_pays(t, x->size(0), x->size(1), sl.r_max, sl.n, sl.tiles(), stream_of(x->device())));
-  });
-}
-
-// set_library(addresses, launch_error, meta_type, plan_long_rows): the
-// library's functions in the order of the struct Library.
+// set_library(addresses, launch_error, meta_type): the library's functions in
+// the order of the struct Library.
 PyObject* py_set_library(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (!arity(n, 4)) return nullptr;
+  if (!arity(n, 3)) return nullptr;
   constexpr int kFns = 11;
   void* p[kFns];
   if (!PyTuple_CheckExact(args[0]) || PyTuple_GET_SIZE(args[0]) != kFns) {
@@ -612,8 +553,6 @@ PyObject* py_set_library(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return nullptr;
     }
   }
-  plan_long_rows = PyLong_AsLongLong(args[3]);
-  if (PyErr_Occurred()) return nullptr;
   lib.last_error = reinterpret_cast<decltype(lib.last_error)>(p[0]);
   lib.shrink_ws = reinterpret_cast<decltype(lib.shrink_ws)>(p[1]);
   lib.shrink = reinterpret_cast<decltype(lib.shrink)>(p[2]);
@@ -644,7 +583,6 @@ PyMethodDef methods[] = {
     MLORA_METHOD("sgemm_b", py_sgemm_b, "(mid, weights, meta, out) -> True, or None"),
     MLORA_METHOD("rmsnorm", py_rmsnorm, "(x, weight, eps) -> new tensor, or None"),
     MLORA_METHOD("add_rmsnorm", py_add_rmsnorm, "(x, residual, weight, eps) -> new tensor, or None"),
-    MLORA_METHOD("planned_pays", py_planned_pays, "(meta, x, a_stacks, b_stacks) -> bool"),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", "Native form of the entry points' ordinary calls.", -1, methods,
                       nullptr,               nullptr,  nullptr,                                            nullptr};
@@ -658,7 +596,7 @@ PyMODINIT_FUNC PyInit__calls() {
   } names[] = {{&s_bs, "bs"},           {&s_max_len, "max_len"},       {&s_seg_indptr, "seg_indptr"},
                {&s_weight_indices, "weight_indices"}, {&s_lora_ranks, "lora_ranks"}, {&s_scalings, "scalings"},
                {&s_plan, "plan"},       {&s_plan_cap, "plan_cap"},     {&s_plan_entries, "plan_entries"},
-               {&s_table_summary, "table_summary"},   {&s_plan_is_current, "plan_is_current"},
+               {&s_table_summary, "table_summary"},
                {&s_bufs, "bufs"},       {&s_buf, "buf"},               {&s_cuda, "cuda"},
                {&s_get, "get"},         {&s_device, "device"}};
   for (auto& it : names)

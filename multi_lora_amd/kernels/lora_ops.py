@@ -92,10 +92,8 @@ class LinkedWorkspace:
             b[4 * _ffi.WS_WAIT_TICKS:4 * _ffi.WS_WAIT_TICKS + 4].view(torch.int32).fill_(int(ticks))
 
 
-# mlora_grouped_workspace_bytes and mlora_apply_segments_workspace_bytes are
-# host arithmetic of their arguments alone.
+# mlora_grouped_workspace_bytes is host arithmetic of its arguments alone.
 _GROUPED_WS_BYTES: Dict[tuple, int] = {}
-_SEGMENTS_WS_BYTES: Dict[tuple, int] = {}
 
 
 def _default_workspace(device: torch.device, linked: bool = False) -> Workspace:
@@ -257,27 +255,6 @@ def expand(mid: torch.Tensor, b_stacks: Sequence[torch.Tensor], meta: KernelInpu
 
 
 GROUPED_MAX_LEN = 16
-
-
-def planned_pays(meta: KernelInputMetaData, x: torch.Tensor, a_stacks: Sequence[torch.Tensor],
-                 b_stacks: Sequence[torch.Tensor]) -> bool:
-    """Whether a batch with segments of more than 16 rows runs faster through
-    the slot-planned path (``apply_grouped``) than as segments.
-
-    The planned path is one launch (or two) where the segment path is three,
-    but it reads an adapter's A and B again for every 16 rows, so it pays
-    while those reads stay small.  Counted here as the bytes its items ask
-    the L2 for: a shrink item is a 256-wide K chunk of the rows and of A, an
-    expand item 256 columns of B and of the output rows (read and written).
-    Measured (planned vs segments, us, 4096 -> 4096 unless said, one prompt):
-    203 rows at rank 64 (19 MB) 8.8 vs 15.3, at rank 16 (9 MB) 6.1 vs 12.5;
-    400 rows at rank 64 (35 MB) 11.7 vs 16.0; 800 rows at rank 16 (32 MB)
-    10.7 vs 14.2, at rank 64 (70 MB) 20.2 vs 19.0; 1600 rows at rank 16
-    (64 MB) 18.1 vs 17.5; 1088 mixed rows to 6144 columns (108 MB) 27.2 vs
-    24.3; the line is drawn at 56 MB.  Captured calls stay with the segment path, which reads the table
-    itself: a replay follows every rewrite of it.
-    """
-    return bool(_ffi.calls().planned_pays(meta, x, a_stacks, b_stacks))
 
 
 class _DevicePlan:
@@ -472,21 +449,6 @@ def build_plan_device(meta: KernelInputMetaData, num_rows: int, num_slots: int, 
     _ffi.check(rc, "mlora_build_plan")
     del keep
     return plan
-
-
-def reserve_segments(x: torch.Tensor, a_stacks: Sequence[torch.Tensor], meta: KernelInputMetaData,
-                     workspace: Workspace) -> None:
-    """Make ``workspace`` large enough for ``apply_segments`` on this call, as
-    running it would: a warm-up of a batch that the planned path takes leaves
-    the captured call, which runs as segments, nothing to allocate."""
-    key = (x.shape[1], a_stacks[0].shape[1], len(a_stacks), x.shape[0], int(meta.bs), int(meta.max_len),
-           _ffi.dtype_code(x.dtype))
-    need = _SEGMENTS_WS_BYTES.get(key)
-    if need is None:
-        if len(_SEGMENTS_WS_BYTES) >= 4096:  # row counts vary per step: keep the cache bounded
-            _SEGMENTS_WS_BYTES.clear()
-        need = _SEGMENTS_WS_BYTES[key] = _ffi.lib().mlora_apply_segments_workspace_bytes(*key)
-    workspace.get(need, x.device)
 
 
 def apply_segments(x: torch.Tensor, a_stacks: Sequence[torch.Tensor], b_stacks: Sequence[torch.Tensor],
