@@ -29,23 +29,39 @@ from ..batch_info import KernelInputMetaData
 _WORKSPACES: Dict[Tuple[str, int], torch.Tensor] = {}
 
 
+def _grown(nbytes: int, old: Sequence[torch.Tensor]) -> int:
+    """Bytes of the buffer that follows ``old``.  At least twice the largest
+    of them, so that all the buffers a workspace keeps come to less than twice
+    its newest."""
+    return max([nbytes, 1 << 20] + [2 * b.numel() for b in old])
+
+
 class Workspace:
     """Caller-owned scratch (fp32 split sums), grown on demand, reused across calls.
 
     Sequential launches on one stream may share a workspace; launches that
-    overlap on different streams need separate workspaces.
+    overlap on different streams need separate workspaces.  A buffer that a
+    larger one replaces is kept: a graph captured with it still reads and
+    writes it on every replay.
     """
 
     def __init__(self) -> None:
         self.buf: Optional[torch.Tensor] = None
+        self.kept: List[torch.Tensor] = []  # every buffer so far
 
     def get(self, nbytes: int, device: torch.device) -> Tuple[int, int]:
         if nbytes <= 0:
             return 0, 0
-        if self.buf is None or self.buf.numel() < nbytes or self.buf.device != device:
-            size = max(nbytes, 1 << 20)
-            self.buf = torch.zeros(size, dtype=torch.uint8, device=device)
-        return self.buf.data_ptr(), self.buf.numel()
+        buf = self.buf
+        if buf is None or buf.numel() < nbytes or buf.device != device:
+            mine = [b for b in self.kept if b.device == device]
+            if mine and mine[-1].numel() >= nbytes:
+                buf = self.buf = mine[-1]
+            else:
+                buf = torch.zeros(_grown(nbytes, mine), dtype=torch.uint8, device=device)
+                self.kept.append(buf)
+                self.buf = buf
+        return buf.data_ptr(), buf.numel()
 
 
 class LinkedWorkspace:
@@ -55,12 +71,15 @@ class LinkedWorkspace:
     single launch tags the flags its work items publish with the launch's
     dispatch id on its hardware queue, which keeps launches on one stream
     apart without ever clearing the buffer; launches on different streams
-    get separate buffers.  Its header words count K chunks that a work item
-    computed itself after a wait gave up, and plan errors.
+    get separate buffers.  A buffer that a larger one replaces is kept: a
+    graph captured with it still reads and writes it on every replay.  The
+    header words count K chunks that a work item computed itself after a wait
+    gave up, and plan errors.
     """
 
     def __init__(self) -> None:
         self.bufs: Dict[Tuple[int, int], torch.Tensor] = {}  # by (device index, stream handle)
+        self.replaced: List[torch.Tensor] = []
 
     def get(self, nbytes: int, device: torch.device, stream: int) -> Tuple[int, int]:
         key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
@@ -71,15 +90,21 @@ class LinkedWorkspace:
                     "the decode workspace of the capturing stream does not exist yet (or is too small): it would "
                     "be allocated and zero-filled inside the graph; run the same calls once on that stream "
                     "before capturing (torch.cuda.graph(g, stream=s) after running them on s)")
-            buf = self.bufs[key] = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            old = [] if buf is None else [buf]
+            buf = torch.zeros(_grown(nbytes, old), dtype=torch.uint8, device=device)
+            self.replaced += old
+            self.bufs[key] = buf
         return buf.data_ptr(), buf.numel()
+
+    def _all(self) -> List[torch.Tensor]:
+        return list(self.bufs.values()) + self.replaced
 
     def counters(self) -> Tuple[int, int]:
         """(chunks computed after a wait gave up, plan errors) summed over all
         buffers (synchronises).  The first only costs time; the second means a
         table's plan did not fit the call and should stay 0."""
         fb = pe = 0
-        for b in self.bufs.values():
+        for b in self._all():
             h = b[:16].view(torch.int32).cpu()
             fb += int(h[_ffi.WS_FALLBACKS])
             pe += int(h[_ffi.WS_PLAN_ERRORS])
@@ -88,7 +113,7 @@ class LinkedWorkspace:
     def set_wait_ticks(self, ticks: int) -> None:
         """Set the wait limit of every buffer (10 ns ticks; 0 = library default;
         negative = no wait: every expand item computes every K chunk itself)."""
-        for b in self.bufs.values():
+        for b in self._all():
             b[4 * _ffi.WS_WAIT_TICKS:4 * _ffi.WS_WAIT_TICKS + 4].view(torch.int32).fill_(int(ticks))
 
 
