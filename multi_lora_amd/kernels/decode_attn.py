@@ -3,8 +3,9 @@
 ``decode_attention`` covers what ``decoder.Attention`` does for one new token
 per sequence over a ``StaticKV`` layer; ``silu_mul`` its MLP's gate.  Both
 return None (nothing launched) for calls they do not take: other dtypes,
-devices and layouts, and tensors that autograd follows; the caller then runs
-the torch operations.
+devices and layouts, and calls whose operations torch has to see (autograd in
+either mode, tracing and compilation, function transforms, dispatch and
+function modes); the caller then runs the torch operations.
 """
 
 from __future__ import annotations
@@ -12,6 +13,9 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import _ffi
 
@@ -23,9 +27,24 @@ _DTYPES = (torch.float16, torch.bfloat16)
 MAX_LEN, MAX_LEN_FEW_HEADS, FEW_HEADS = 2048, 1024, 64
 
 
+def _followed() -> bool:
+    """Whether something follows the torch operations run now: a launch past
+    torch would drop out of it (a forward-mode tangent, a recorded graph, a
+    batched dimension), although its tensors look plain."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or (torch._C._len_torch_function_stack() > 0
+                and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())))
+
+
 def _plain(*tensors: torch.Tensor) -> bool:
+    if _followed():
+        return False
     first = tensors[0]
-    return (first.is_cuda and first.dtype in _DTYPES
+    # A launch goes to the current device; torch's operations follow the tensor.
+    return (first.is_cuda and first.dtype in _DTYPES and first.device.index == torch.cuda.current_device()
             and all(type(t) is torch.Tensor and t.device == first.device for t in tensors)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
@@ -60,6 +79,8 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
         return None
     if pos.dtype != torch.int64 or pos.numel() != 1 or values.data_ptr() % 16:
         return None
+    if (keys.is_inference() or values.is_inference()) and not torch.is_inference_mode_enabled():
+        return None  # torch refuses the write
     out = torch.empty((b, heads * d), dtype=q.dtype, device=q.device)
     rc = _ffi.lib().mlora_decode_attention(
         q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), cos.data_ptr(), sin.data_ptr(),
@@ -69,6 +90,8 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
     if rc == -2:
         return None
     _ffi.check(rc, "mlora_decode_attention")
+    # Written in place: a backward pass that saved the caches must notice.
+    torch.autograd.graph.increment_version((keys, values))
     return out
 
 

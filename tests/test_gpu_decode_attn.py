@@ -4,7 +4,11 @@ every head grouping, strided inputs, and calls it leaves to torch."""
 
 import pytest
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
+from multi_lora_amd.decoder import MLP, Attention, DecoderConfig, Rotary, StaticKV
 from multi_lora_amd.kernels.decode_attn import decode_attention, silu_mul
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +87,113 @@ def test_silu_mul(dev, shape, dtype):
     assert got.shape == gate.shape and got.is_contiguous()
     torch.testing.assert_close(got.double(), want, rtol=2.0 ** (-8 if dtype == torch.bfloat16 else -11), atol=1e-6)
     assert silu_mul(gate.float(), up.float()) is None and silu_mul(gate[..., :-1], up[..., :-1]) is None
+
+
+CONFIG = DecoderConfig(hidden_size=256, intermediate_size=512, num_attention_heads=4, num_key_value_heads=2)
+POS = 5
+
+
+def layer(dev, kind):
+    """One decode step through the decoder's module ``kind``, as a function of its input."""
+    torch.manual_seed(3)
+    if kind == "mlp":
+        return MLP(CONFIG).to(dev, torch.bfloat16).requires_grad_(False)
+    attn = Attention(CONFIG).to(dev, torch.bfloat16).requires_grad_(False)
+    inv = 1.0 / (CONFIG.rope_theta ** (torch.arange(0, 64, 2, device=dev) / 64))
+    rot = Rotary.make(torch.full((3,), POS, device=dev), inv, torch.bfloat16)
+    hide = (torch.arange(8, device=dev) > POS).view(1, 1, 1, 8).expand(3, 1, 1, 8)
+    filled = [torch.randn(3, 2, 64, 8, device=dev).bfloat16(), torch.randn(3, 2, 8, 64, device=dev).bfloat16()]
+    at = torch.tensor([POS], device=dev)
+
+    def run(x):
+        kv = StaticKV(CONFIG, 3, 8, dev, torch.bfloat16)
+        kv.keys[0].copy_(filled[0])
+        kv.values[0].copy_(filled[1])
+        return attn(x, rot, hide, kv, 0, at)
+
+    return run
+
+
+def rows(dev, seed):
+    return torch.randn(3, 1, 256, generator=torch.Generator().manual_seed(seed)).bfloat16().to(dev)
+
+
+def close(got, want):
+    torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("kind", ["mlp", "attention"])
+def test_forward_mode_keeps_the_tangent(dev, kind, grad):
+    f, x, t = layer(dev, kind), rows(dev, 1), rows(dev, 2)
+    with torch.set_grad_enabled(grad):
+        with forward_ad.dual_level():
+            out = forward_ad.unpack_dual(f(forward_ad.make_dual(x, t)))
+        assert out.tangent is not None
+        step = 0.125  # a power of two: x +- step * t differ from x by few roundings
+        want = (f(x + step * t).float() - f(x - step * t).float()) / (2 * step)
+    close(out.primal, f(x))
+    assert (out.tangent.float() - want).norm() <= 0.1 * want.norm()
+
+
+def test_function_transforms_and_traces_see_torch_operations(dev):
+    f, x, t = layer(dev, "mlp"), rows(dev, 1), rows(dev, 2)
+    want = f(x)
+    close(torch.func.vmap(f)(x), want)
+    assert bool(torch.func.jvp(f, (x,), (t,))[1].any())
+    traced = torch.jit.trace(f, (t,), check_trace=False)
+    close(traced(x), want)
+    attn = layer(dev, "attention")
+    close(torch.jit.trace(attn, (t,), check_trace=False)(x), attn(x))
+
+
+class Counting(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+class CountingFunctions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(getattr(func, "__name__", ""))
+        return func(*args, **(kwargs or {}))
+
+
+def test_modes_see_torch_operations_and_a_default_device_does_not_matter(dev):
+    gate, up = rows(dev, 1), rows(dev, 2)
+    f, x = layer(dev, "mlp"), rows(dev, 1)
+    with Counting() as mode:
+        f(x)
+    assert any("silu" in s for s in mode.seen)
+    with CountingFunctions() as mode:
+        f(x)
+    assert any("silu" in s for s in mode.seen)
+    with torch.device(dev):
+        assert silu_mul(gate, up) is not None
+
+
+def test_calls_of_another_device_than_the_current_one_are_left_to_torch(dev, monkeypatch):
+    gate, up = rows(dev, 1), rows(dev, 2)
+    assert silu_mul(gate, up) is not None
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert silu_mul(gate, up) is None
+
+
+def test_the_cache_write_is_counted_and_inference_caches_stay_refused(dev):
+    args = inputs(dev, 2, 4, 2, 64, 40, torch.bfloat16, 0, 1)
+    at = torch.tensor([3], device=dev)
+    before = args[5]._version, args[6]._version
+    assert decode_attention(*args, at, 0.125) is not None
+    assert args[5]._version > before[0] and args[6]._version > before[1]
+    with torch.inference_mode():
+        made = inputs(dev, 2, 4, 2, 64, 40, torch.bfloat16, 0, 1)
+        assert decode_attention(*made, at, 0.125) is not None
+    assert decode_attention(*made, at, 0.125) is None
