@@ -348,9 +348,10 @@ int mlora_pool_scatter(const void* stage, int64_t stage_row_stride, int32_t h, c
  * (x * cos + roll(x, D / 2) * sin, cos and sin [batch or 1, D] of the data
  * dtype, row stride rot_row_stride, 0 to share one row), k and v go into
  * keys [batch, kv_heads, D, len] and values [batch, kv_heads, len, D] at
- * position *pos (device memory, int64; outside [0, len) nothing is written),
- * and out [batch, heads * D] = softmax(scale * q . keys, positions with a
- * nonzero hide[batch or 1, len] byte left out) . values, fp32 math.
+ * position *pos (device memory, int64; outside [0, len) neither is written
+ * and out is NaN), and out [batch, heads * D] = softmax(scale * q . keys,
+ * positions with a nonzero hide[batch or 1, len] byte left out) . values,
+ * fp32 math.
  * Requirements (else -2): bf16 or fp16; D 64 or 128; heads / kv_heads 1, 2, 4
  * or 8; len <= 2048; values 16-byte aligned.
  * No counterpart is called in the reference (its model runs its own

@@ -239,7 +239,9 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(AttnArgs a) {
     float f = 0.f;
 #pragma unroll
     for (int w = 0; w < kAttnWaves; ++w) f += s.out[w][r][e];
-    out[i] = T::from_f32(f);
+    // A position outside the cache: the token's key and value have no place,
+    // and attention without them is no answer.
+    out[i] = T::from_f32(pos >= 0 ? f : NAN);
   }
 }
 

@@ -55,7 +55,9 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
     """Rotary on ``q [b, heads*d]`` and ``k [b, kv_heads*d]``, the new key and
     value into ``keys [b, kv_heads, d, L]`` / ``values [b, kv_heads, L, d]`` at
     ``pos`` (one int64 on the device), and the attention of every row over the
-    cache, except the positions ``hide [b, 1, 1, L]`` marks; ``[b, heads*d]``."""
+    cache, except the positions ``hide [b, 1, 1, L]`` marks; ``[b, heads*d]``.
+    A ``pos`` outside the cache, which only the device knows, writes nothing
+    and makes the result NaN."""
     if not _plain(q, k, v, cos, sin, keys, values, hide, pos) or values.dim() != 4:
         return None
     b, kv_heads, length, d = values.shape

@@ -67,8 +67,8 @@ def test_decode_attention(dev, b, heads, kv_heads, d, length, pad, dtype):
 def test_decode_attention_positions_and_refusals(dev):
     args = inputs(dev, 2, 4, 2, 64, 40, torch.bfloat16, 0, 1)
     keys, values = args[5].clone(), args[6].clone()
-    for pos in (-1, 40):                                  # outside the cache: nothing is written
-        assert decode_attention(*args, torch.tensor([pos], device=dev), 0.125) is not None
+    for pos in (-1, 40):                                  # outside the cache: nothing is written, no answer
+        assert bool(decode_attention(*args, torch.tensor([pos], device=dev), 0.125).isnan().all())
     assert torch.equal(args[5], keys) and torch.equal(args[6], values)
     at = torch.tensor([3], device=dev)
     assert decode_attention(*[t.float() if t.dtype == torch.bfloat16 else t for t in args], at, 0.125) is None
