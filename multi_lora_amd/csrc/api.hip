@@ -94,6 +94,19 @@ size_t mid_region_bytes(int32_t rows, int32_t n_slices, int32_t r_max, int32_t d
   return (b + 255) / 256 * 256;
 }
 
+// Bytes of split sums the shrink needs, whether or not the call's rows turn
+// out to be made of 16-byte chunks.  False: unsupported shape.
+bool shrink_ws_bytes(int32_t in_dim, int32_t r_max, int32_t n_slices, int32_t num_rows, int32_t bs, int32_t max_len,
+                     int32_t dtype, size_t* bytes) {
+  *bytes = 0;
+  for (const bool aligned : {true, false}) {
+    mlora::ShrinkPlan p;
+    if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, aligned, num_cus(), &p)) return false;
+    *bytes = std::max(*bytes, p.ws_bytes);
+  }
+  return true;
+}
+
 // Whether every row the shrink reads is made of 16-byte chunks.
 bool shrink_aligned(const void* x, int64_t x_row_stride, int32_t in_dim, const mlora_slice* slices, int32_t n_slices,
                     int32_t dtype) {
@@ -240,9 +253,8 @@ const char* mlora_last_error(void) { return g_err; }
 size_t mlora_shrink_workspace_bytes(int32_t in_dim, int32_t r_max, int32_t n_slices, int32_t num_rows, int32_t bs,
                                     int32_t max_len, int32_t dtype) {
   if (!valid_dtype(dtype)) return 0;
-  mlora::ShrinkPlan p;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, true, num_cus(), &p)) return 0;
-  return p.ws_bytes;
+  size_t bytes;
+  return shrink_ws_bytes(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, &bytes) ? bytes : 0;
 }
 
 int mlora_shrink(const void* x, int64_t x_row_stride, int32_t num_rows, int32_t in_dim, const mlora_slice* slices,
@@ -265,9 +277,9 @@ int mlora_expand(const void* mid, int64_t mid_row_stride, int32_t num_rows, cons
 size_t mlora_apply_segments_workspace_bytes(int32_t in_dim, int32_t r_max, int32_t n_slices, int32_t num_rows,
                                             int32_t bs, int32_t max_len, int32_t dtype) {
   if (!valid_dtype(dtype) || num_rows < 0 || r_max <= 0 || n_slices < 1) return 0;
-  mlora::ShrinkPlan p;
-  if (!mlora::plan_shrink(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, true, num_cus(), &p)) return 0;
-  return mid_region_bytes(num_rows, n_slices, r_max, dtype) + p.ws_bytes;
+  size_t bytes;
+  if (!shrink_ws_bytes(in_dim, r_max, n_slices, num_rows, bs, max_len, dtype, &bytes)) return 0;
+  return mid_region_bytes(num_rows, n_slices, r_max, dtype) + bytes;
 }
 
 int mlora_apply_segments(const void* x, int64_t x_row_stride, int32_t num_rows, int32_t in_dim,

@@ -59,8 +59,7 @@ struct ShrinkPlan {
   size_t ws_bytes;
 };
 
-// aligned: every operand row is readable as 16-byte chunks.  A plan of
-// unaligned rows needs no more workspace than the aligned one.
+// aligned: every operand row is readable as 16-byte chunks.
 bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, bool aligned,
                  int num_cus, ShrinkPlan* plan);
 // Launches the shrink and, when K is split, the in-order split reduction.

@@ -13,14 +13,14 @@
 //   short segments (<= 16 rows, shrink_kernel): workgroup = (segment, K
 //     split); the 4 waves take alternate K-steps of the same 16 rows and are
 //     summed through LDS in wave order.
-//   calls whose tiles are few or small, unaligned 16-bit rows, most fp32:
-//     workgroup = 16-row tile over the whole reduction (shrink_wide.hip).
+//   calls whose tiles read little, most unaligned and fp32 calls: workgroup =
+//     16-row tile over the whole reduction (shrink_wide.hip; wide_pays).
 //   long segments: workgroup = (dense 64-row tile, K split); each wave owns
 //     16 rows of the tile and every rank block.  16-bit aligned data with K
 //     splits in multiples of 64 stream x and A straight into LDS three
 //     stages deep (shrink_dma_kernel); other 16-bit aligned data stage them
-//     through registers (shrink_lds_kernel); fp32 and more than eight A
-//     blocks load MFMA fragments directly (shrink_rows_kernel).
+//     through registers (shrink_lds_kernel); unaligned rows, fp32 and more
+//     than eight A blocks load MFMA fragments directly (shrink_rows_kernel).
 // When K is split over workgroups each split stores fp32 sums and a second
 // launch adds them in split order, so the result is deterministic and no
 // workgroup ever waits on another.
@@ -832,9 +832,7 @@ hipError_t launch_nbt_al(const ShrinkPlan& p, const ShrinkArgs& args, hipStream_
   if (p.bm != 64 * RB) return hipErrorInvalidValue;
   if constexpr (AL && sizeof(typename T::raw_t) == 2 && NBT <= 8)
     return launch_with<T>(shrink_lds_kernel<T, NBT, RB>, p, args, stream);
-  // Unaligned 16-bit rows of up to eight blocks are the wide kernel's.
-  if constexpr (!AL && sizeof(typename T::raw_t) == 2 && NBT <= 8) return hipErrorInvalidValue;
-  else return launch_with<T>(shrink_rows_kernel<T, NBT, RB, AL>, p, args, stream);
+  return launch_with<T>(shrink_rows_kernel<T, NBT, RB, AL>, p, args, stream);
 }
 
 template <class T, bool AL>
@@ -878,30 +876,49 @@ hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, int dtype, 
 }  // namespace
 
 // Whether the shrink runs as one launch of 16-row tiles over the whole
-// reduction (shrink_wide.hip) rather than split over workgroups.  A CU loads
-// such a tile's rows (x and every A block) at 60-85 GB/s, so what counts is
-// the bytes a CU loads, tile after tile.  Measured (whole calls, us, split vs
-// wide):
-//   16-bit, 4096 wide, rank 8 / 32 / 64 (256 / 384 / 640 KB a tile): 60 rows
-//     11.0 / 11.8 / 14.9 vs 10.2 / 11.6 / 15.6; 600 rows 13.8 / 14.5 / 18.2 vs
-//     12.3 / 13.7 / 19.8; 3900 rows 24.2 / 26.5 / 33.7 vs 21.7 / 24.1 / 31.1;
-//     1088 mixed rows to q|k|v at rank 16 (512 KB) 24.3 vs 24.7;
-//   unaligned 16-bit rows, which have no other staged form: K 4101, 4075 rows
-//     at rank 64 93.6 vs 40.6; K 14001, 958 rows at rank 64 (2.2 MB) 74.4 vs
-//     60.6; K 1001, 300 rows 27.0 vs 18.6;
-//   fp32: 958 rows at rank 16 (512 KB) 23.9 vs 21.1, rank 64 (1.3 MB) 43.5 vs
-//     44.9; 4075 rows, two slices at rank 64 (2.3 MB) 184.7 vs 129.1;
-//   decode-shaped calls (no segment over 16 rows: the split's expand adds the
-//     sums itself): fp32, 128 rows at rank 16 25.9 vs 22.6, 256 rows to q|k|v
-//     at rank 32 282 vs 104, but 8 rows 10.8 vs 13.8; K 4101, 64 rows 13.2 vs
-//     15.4.
-bool wide_pays(int in_dim, int launch_blocks, int blocks, int tiles, int max_len, int dtype, bool aligned, int num_cus) {
-  if (max_len <= 16 && tiles < num_cus / 2) return false;
+// reduction (shrink_wide.hip) rather than split over workgroups.  What counts
+// is the bytes a tile reads, its 16 rows of x and every A block over all of K,
+// which one CU loads, and how full the tiles are: a one-row segment reads as
+// much as a 16-row one.  Measured on 1,360 whole calls, cold inputs, K 255 to
+// 14336, ranks 8 to 128, 17 to 4075 rows (time as wide / time as split, by
+// bytes a tile):
+//   16-bit, segments of 64 rows and more on average: up to 192 KB 0.69-1.01,
+//     256 KB 0.84-0.93 on up to 133 tiles but 1.00-1.05 on 247, 384 KB
+//     0.92-1.06.  Shorter and mixed segments, whose expand adds the split's
+//     sums itself (no reduce launch): up to 160 KB 0.74-1.02, 192 KB up to
+//     1.07, 256 KB 1.12, 384 KB 1.26 (2 x 512 + 64 rows, the bench's o call at
+//     256 KB: 16.8 split, 18.5 wide).
+//   No segment over 16 rows (r_max the planned path does not take): up to 96 KB
+//     0.85-1.03; one or two A blocks of 128-384 KB 1.00-1.13 on 128 tiles,
+//     0.80-0.96 on 200; four and more up to 400 KB 0.41-0.51.
+//   Unaligned 16-bit rows, whose split loads them in fragment order: up to 160
+//     KB 0.44-0.97; past that 0.40-0.99 (0.44-1.04 up to K 8193) when the tiles
+//     are full, there are several A blocks or half the chip has a tile, but 17
+//     rows 0.8-1.8 and K 14001 over few tiles 1.0-1.5.  No segment over 16 rows:
+//     0.45-0.96 once every CU has a tile, less than half the chip 0.7-1.9.
+//   fp32: up to 640 KB 0.52-0.97; past that on half the chip's tiles 0.56-0.99
+//     (1.02-1.08 with mostly one-row tiles of 1.8 MB), on fewer up to 1.9.  No
+//     segment over 16 rows: 0.32-1.01 on half the chip's tiles.
+bool wide_pays(int in_dim, int launch_blocks, int blocks, int rows, int bs, int tiles, int max_len, int dtype,
+               bool aligned, int num_cus) {
   const int64_t bytes = static_cast<int64_t>(launch_blocks + 1) * 16 * in_dim * (dtype == MLORA_F32 ? 4 : 2);
-  if (dtype == MLORA_F32) return bytes <= (1100 << 10) || tiles >= num_cus / 2;
-  if (!aligned) return true;
+  const bool half = tiles >= num_cus / 2;
+  const bool full = rows >= 12LL * tiles;
+  const bool decode = max_len <= 16;
+  if (dtype == MLORA_F32) return decode ? half : bytes <= (640 << 10) || (half && (full || bytes <= (1100 << 10)));
+  if (!aligned) {
+    if (decode) return bytes >= (32 << 10) && (tiles >= num_cus || (half && launch_blocks >= 4));
+    if (bytes <= (160 << 10)) return true;
+    if (in_dim > 10240) return half && (full || launch_blocks >= 2);
+    return rows >= 32 && (full || half || launch_blocks >= 2);
+  }
+  if (blocks != launch_blocks) return false;
   const int64_t rounds = (static_cast<int64_t>(tiles) + num_cus - 1) / num_cus;
-  return blocks == launch_blocks && bytes * rounds <= (400 << 10);
+  if (decode)
+    return half && bytes * rounds <= (400 << 10) &&
+           (launch_blocks >= 4 || bytes <= (96 << 10) || tiles >= num_cus * 3 / 4);
+  const bool long_segments = rows >= 64LL * bs;
+  return bytes * rounds <= (!long_segments ? 160 << 10 : tiles <= num_cus * 3 / 4 ? 256 << 10 : 192 << 10);
 }
 
 bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_len, int dtype, bool aligned,
@@ -921,7 +938,7 @@ bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_
   if (p.nbt > 16) return false;
   const int tiles16 = static_cast<int>(std::min<int64_t>(
       dense_tiles(bs, cdiv(max_len > 0 ? max_len : 1, 16), rows, 16), INT32_MAX));
-  if (p.nbt <= 8 && wide_pays(in_dim, blocks, n_slices * per_slice, tiles16, max_len, dtype, aligned, num_cus)) {
+  if (p.nbt <= 8 && wide_pays(in_dim, blocks, n_slices * per_slice, rows, bs, tiles16, max_len, dtype, aligned, num_cus)) {
     p.wide = 1;
     p.bm = 16;
     p.m_tiles = cdiv(max_len > 0 ? max_len : 1, p.bm);
@@ -967,7 +984,7 @@ bool plan_shrink(int in_dim, int r_max, int n_slices, int rows, int bs, int max_
     // (22.5 vs 22.0 us), and batches of short segments keep 64 rows.  At
     // most four A blocks a launch: with eight, three 128-row stages need
     // 96 KB of LDS, one workgroup a CU.
-    if (streamed && in_dim >= kLongKRows128 && rows >= 256LL * bs && p.nbt <= 4) {
+    if (streamed && aligned && in_dim >= kLongKRows128 && rows >= 256LL * bs && p.nbt <= 4) {
       p.bm = 128;
       p.m_tiles = cdiv(max_len > 0 ? max_len : 1, p.bm);
     }

@@ -13,11 +13,12 @@
 // 30 GB/s of L2 hits this way; in row order, 60-85 GB/s measured in this
 // kernel (one 1000-row prompt, 4096 -> 4096 at rank 64, shrink: 25.9 -> 11.6
 // us).  It is bound by that rate: a tile reads its x rows and its adapter's
-// whole A, (A blocks + 1) * 16 rows of K.  Measured against the split kernels
-// (whole calls, us): 8 prompts of 4075 rows, 4096 -> 4096 at rank 8, 24.2 ->
-// 21.7; 600 rows, 1024 -> 4096 at rank 64, 17.4 -> 13.9; fp32 rows 5, 17 and
-// 42, 1024 -> 1024 at rank 8, 13.3 -> 8.9; 958 rows of K 4101, rank 16, 24.3
-// -> 18.5.  wide_pays (shrink.hip) has the line.
+// whole A, (A blocks + 1) * 16 rows of K.  Whole calls against the split
+// kernels (us, cold inputs): a prompt of 203 rows, 4096 -> 4096 at rank 16,
+// 13.5 -> 11.4; 600 rows, 1024 -> 4096 at rank 64, 18.5 -> 15.2; fp32 rows 5, 17
+// and 42, 1024 -> 1024 at rank 8, 16.9 -> 9.9; 7 prompts of 300 rows of K 4101 at
+// rank 64, 70 -> 36; q|k|v of 256 fp32 rows at rank 32, 256 -> 88.  wide_pays
+// (shrink.hip) has the line.
 #include "kernels.h"
 #include "loads.h"
 

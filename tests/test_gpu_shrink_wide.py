@@ -61,3 +61,14 @@ def test_unaligned_rows(dev, in_dim, pad, dtype):
 
 def test_many_one_row_segments_in_fp32(dev):
     run(dev, 520, 2, 16, torch.float32, ranks=[16, 8, 0, 3], lens=[1] * 150, slots=[i % 4 for i in range(150)])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("in_dim,r_max,pad,lens", [(4101, 8, 0, [17]), (14001, 64, 0, [20, 1]), (14336, 16, 4, [300])])
+def test_unaligned_rows_of_few_tiles_are_split(dev, in_dim, r_max, pad, lens, dtype):
+    # The last shape plans 128-row tiles when its rows are aligned.
+    run(dev, in_dim, 1, r_max, dtype, pad=pad, ranks=[r_max, 5], lens=lens, slots=list(range(len(lens))))
+
+
+def test_unaligned_decode_rows_get_the_workspace_they_need(dev):
+    run(dev, 4096, 1, 20, torch.bfloat16, pad=4, ranks=[20, 9, 0, 17], lens=[1] * 200, slots=[i % 4 for i in range(200)])
