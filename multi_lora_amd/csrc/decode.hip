@@ -10,8 +10,8 @@
 //
 //   shrink item  (entry, slice group, K chunk of 4 waves x SP x 32): the
 //                entry (with its rows) comes in one scalar load, then the
-//                chunk's A rows and the entry's x rows go to LDS together;
-//                they are multiplied on MFMA (16 rank rows x 16 token rows a
+//                chunk's A fragments and the entry's x rows together; they
+//                are multiplied on MFMA (16 rank rows x 16 token rows a
 //                tile), the four waves' sums added in LDS, and the chunk's
 //                fp32 sums stored to the workspace.
 //   expand item  (entry, 256 output columns of one slice): B fragments and
@@ -48,12 +48,10 @@
 //
 // Two launches: shrink items, then expand items, with the same bodies and
 // the same sums (bit-identical results); the kernel boundary orders them.
-// Grids of more than kDirectItems shrink items run an entry's items next to
-// each other (item_fast), so the workgroups in flight read whole A rows and
-// neighbouring B rows; with the entry fastest they all read at one offset of
-// their rows (a layer's calls for 77 rows over 40 adapters: 113.4 -> 110.3 us;
-// RMSNorm + q|k|v for 256 rows: 40.9 -> 40.4).  Smaller grids keep an entry
-// on one XCD, whose L2 then still holds its sums.
+// Large grids run an entry's items next to each other (ITEM_FAST), so the
+// workgroups in flight read whole A rows and neighbouring B rows; with the
+// entry fastest they all read at one offset of their rows.  Smaller grids keep
+// an entry on one XCD, whose L2 then still holds its sums (orders_of).
 //
 // Fused RMSNorm (two launches): the shrink launch also holds the RMSNorm of
 // the call's rows (the RMSNorm kernel's row body, so the same y, and each
@@ -127,9 +125,9 @@ __device__ uint64_t planned_dispatch_id() __asm("llvm.amdgcn.dispatch.id");
 namespace {
 
 constexpr int kDefaultWaitTicks = 20000;  // 200 us of s_memrealtime (100 MHz)
-// Two-launch grids of up to this many shrink items (four workgroups a CU) run
-// at once, bound by one workgroup's latency.
-constexpr int64_t kDirectItems = 1024;
+// Two-launch shrink grids of up to this many A blocks (items times blocks an
+// item) run about at once, bound by one workgroup's latency.
+constexpr int64_t kDirectBlocks = 1024;
 constexpr int kGroups = 4;                // chunk groups summed separately, then in order
 
 struct Entry {
@@ -197,49 +195,29 @@ __device__ __forceinline__ const R* a_block_row(const DecodeArgs& a, const Entry
   return slice_a<R>(a.slices, s_first + sl, en.slot, min((j - sl * nb_act) * 16 + r, en.rank - 1));
 }
 
-// Bytes of LDS a wave stages a K chunk's rows in: SP K-steps (128 bytes) of 16
-// rows of every A block and of x.
-template <int NBT, int SP>
-constexpr int kStageBytes = (NBT + 1) * 16 * SP * 64;
-
-typedef __attribute__((address_space(1))) void gvoid_t;
-typedef __attribute__((address_space(3))) void lvoid_t;
-
 // One K chunk of one entry's shrink, for the slices of group sg:
 // sums[i][n] = sum over the chunk of x[row_i, k] * A_s[slot, n, k], stored to
 // the workspace by wave 0 for the entry's rows, then (flag != 0) the chunk's
-// flag once the sums are acknowledged.  All threads call it; it ends with an
-// LDS barrier.  Wave w takes SP neighbouring K-steps of the chunk.
+// flag once the sums are acknowledged.  xrow: this lane's x row (row
+// lane & 15 of the entry).  red: 3 * NBT * 64 vectors of LDS.  All threads
+// call it; it ends with an LDS barrier.
 //
-// kStaged (the two-launch schedule, and the single launch over four A blocks
-// at r_max 64): the wave's rows go from memory to its own part of `stage` with eight neighbouring lanes on a row's 128
-// bytes, and the MFMA fragments are read from there.  Loaded in fragment
-// order (lane l on row l % 16), every four neighbouring lanes ask for four
-// cache lines, and the CU's vector memory path takes about 4 times as long
-// per instruction: 38 GB/s a CU against 122-128 (1 MB in the L2, all CUs
-// reading), 9.6 TB/s over the chip with every L2 hit counted.  LDS row r
-// holds source chunk c ^ (r >> 1 & 7) at chunk c, which spreads a fragment
-// read over the banks.  The single launch of o and down for 77 rows at r_max
-// 64: 18.7 -> 17.4 us on average; the shrink half of RMSNorm + q|k|v, 22 us,
-// is bound by its dependent round trips and stays.  xr: x rows (lane / 8) and 8 + lane / 8 of the entry.
-//
-// kDirect (the other single launches, whose few workgroups are bound by one
-// workgroup's latency: a decoder's step of sixteen calls 684 us, 688 staged):
-// every fragment requested at once, in registers.  kLean (the expand items'
-// rare recompute): one A block's at a time, so that the launch keeps its
-// occupancy.  The same products in the same order, so the same sums in every
-// form.  xr[0]: x row lane % 16 of the entry.
-//
+// Every fragment of the chunk is requested at once, in registers; blocks past
+// the entry's rank are not loaded (q|k|v of 256 rows over 112 adapters of
+// ranks 8 to 64 in r_max 64: shrink 29.9 -> 22.5 us, with the grid order).  A's
+// rows staged through LDS in row order (eight neighbouring lanes to 128 bytes,
+// 3 times the L1 rate) are slower, staged / direct: the same call 25.9 / 22.5,
+// rank 64 39.4 / 36.3, rank 32 22.3 / 20.4, rank 8 11.3 / 8.8, and in the single
+// launch 2-5 %; the LDS keeps workgroups off the CU.
+// LEAN: one A block's fragments in flight at a time (the same products in the
+// same order, so the same sums), for the expand items' rare recompute, so
+// that the single launch keeps its occupancy.
 // NORM (the fused RMSNorm launch): the MFMA takes round(x * w) with the
 // RMSNorm weight nw.
-// red(w): where wave w (1..3) leaves its sums for wave 0.
-enum class Form { kStaged, kDirect, kLean };
-
-template <class T, int NBT, int SP, Form FORM, bool NORM = false, class Red>
-__device__ void shrink_chunk(const DecodeArgs& a, int e, const Entry& en, const int (&xr)[2], int sg, int c, Red red,
-                             uint64_t flag, unsigned char* stage, const typename T::raw_t* nw = nullptr) {
-  static_assert(!NORM || FORM != Form::kLean, "the fused RMSNorm path has no recompute");
-  static_assert(SP == 2, "a wave's K-steps are 128 bytes of a row");
+template <class T, int NBT, int SP, bool LEAN, bool NORM>
+__device__ void shrink_chunk(const DecodeArgs& a, int e, const Entry& en, int xrow, int sg, int c, f32x4* red,
+                             uint64_t flag, const typename T::raw_t* nw) {
+  static_assert(!(NORM && LEAN), "the fused RMSNorm shrink has no recompute path");
   using raw = typename T::raw_t;
   constexpr int VEC = T::VEC;
   constexpr int KSTEP = T::KSTEP;
@@ -251,125 +229,83 @@ __device__ void shrink_chunk(const DecodeArgs& a, int e, const Entry& en, const 
   const int nb_act = (en.rank + 15) >> 4;
   const int s_first = (a.s_groups == 1) ? 0 : sg;
   const int nbt = ((a.s_groups == 1) ? a.n_slices : 1) * nb_act;
-  const int kw = c * a.k_chunk + wave * SP * KSTEP;
+  // Element of K-step sp of this lane's fragments.  Loads are unmasked (clamped
+  // in bounds) and dropped past in_dim where the MFMA uses them; in_dim is a
+  // multiple of the 16-byte chunk: one is wholly inside or wholly outside.
+  auto k_of = [&](int sp) { return c * a.k_chunk + (wave * SP + sp) * KSTEP + g * VEC; };
 
-  // Rows are read unmasked (clamped in bounds) and dropped past in_dim where
-  // the MFMA uses them.  in_dim is a multiple of the chunk: a chunk is wholly
-  // inside or wholly outside.
   f32x4 acc[NBT];
 #pragma unroll
   for (int j = 0; j < NBT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto load_w = [&](u32x4 (&wv)[SP]) {
+  auto load_a = [&](int j, u32x4 (&af)[SP]) {
+    const int sl = j / nb_act;  // slice within the group
+    const raw* arow = slice_a<raw>(a.slices, s_first + sl, en.slot, min((j - sl * nb_act) * 16 + r16, en.rank - 1));
+#pragma unroll
+    for (int sp = 0; sp < SP; ++sp) af[sp] = ld_chunk(arow + (k_of(sp) < a.in_dim ? k_of(sp) : 0));
+  };
+  auto load_x = [&](u32x4 (&xv)[SP]) {
+    const raw* row = static_cast<const raw*>(a.x) + static_cast<int64_t>(xrow) * a.x_stride;
 #pragma unroll
     for (int sp = 0; sp < SP; ++sp) {
-      const int kk = kw + sp * KSTEP + g * VEC;
-      wv[sp] = ld_chunk(nw + (kk < a.in_dim ? kk : 0));
+      const u32x4 v = ld_chunk(row + (k_of(sp) < a.in_dim ? k_of(sp) : 0));
+      xv[sp] = k_of(sp) < a.in_dim ? v : zero_chunk();
     }
   };
-  auto weigh = [&](const u32x4& x, const u32x4& w) {
-    float f[VEC];
+  auto mma_a = [&](int j, const u32x4 (&af)[SP], const u32x4 (&xv)[SP]) {
 #pragma unroll
-    for (int q = 0; q < VEC; ++q) f[q] = chunk_elem<T>(x, q) * chunk_elem<T>(w, q);
-    return pack_chunk<T>(f);
+    for (int sp = 0; sp < SP; ++sp) acc[j] = T::mma(acc[j], k_of(sp) < a.in_dim ? af[sp] : zero_chunk(), xv[sp]);
   };
-  if constexpr (FORM == Form::kStaged) {
-    unsigned char* mine = stage + wave * kStageBytes<NBT, SP>;
-    const int r8 = lane >> 3;
-    // Instruction i of a block fills its rows 8 i .. 8 i + 7.
-    auto fill = [&](int blk, int i, const raw* row) {
-      const int kk = kw + (((lane & 7) ^ (((8 * i + r8) >> 1) & 7)) << 3);
-      __builtin_amdgcn_global_load_lds((gvoid_t*)(row + (kk < a.in_dim ? kk : 0)),
-                                       (lvoid_t*)(mine + (blk * 2 + i) * 1024), 16, 0, 0);
-    };
+  u32x4 xv[SP];
+  if constexpr (!LEAN) {
+    // x before A: its address waits for the row word, and a wait among the A
+    // loads, whose number depends on the rank, would be for all of them.
+    load_x(xv);
+    u32x4 wv[SP];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int sp = 0; sp < SP; ++sp) wv[sp] = ld_chunk(nw + (k_of(sp) < a.in_dim ? k_of(sp) : 0));
+    }
+    u32x4 af[NBT][SP];
+#pragma unroll
+    for (int j = 0; j < NBT; ++j)
+      if (j == 0 || j < nbt) load_a(j, af[j]);
+    fence_regs(af);
+    if constexpr (NORM) {
+#pragma unroll
+      for (int sp = 0; sp < SP; ++sp) {
+        float f[VEC];
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) f[q] = chunk_elem<T>(xv[sp], q) * chunk_elem<T>(wv[sp], q);
+        xv[sp] = k_of(sp) < a.in_dim ? pack_chunk<T>(f) : zero_chunk();
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NBT; ++j)
+      if (j < nbt) mma_a(j, af[j], xv);
+  } else {
+    load_x(xv);
 #pragma unroll
     for (int j = 0; j < NBT; ++j) {
       if (j >= nbt) break;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fill(j, i, a_block_row<raw>(a, en, s_first, nb_act, j, 8 * i + r8));
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) fill(NBT, i, static_cast<const raw*>(a.x) + static_cast<int64_t>(xr[i]) * a.x_stride);
-    u32x4 wv[SP];
-    if constexpr (NORM) load_w(wv);
-    // The wave reads only what it loaded itself: no barrier.
-    asm volatile("" ::: "memory");
-    wait_vmcnt<0>();
-    asm volatile("" ::: "memory");
-    auto frag = [&](int blk, int sp) {
-      return *reinterpret_cast<const u32x4*>(mine + blk * 2048 + r16 * 128 + (((sp * 4 + g) ^ ((r16 >> 1) & 7)) << 4));
-    };
-#pragma unroll
-    for (int sp = 0; sp < SP; ++sp) {
-      const bool in = kw + sp * KSTEP + g * VEC < a.in_dim;
-      u32x4 xv = in ? frag(NBT, sp) : zero_chunk();
-      if constexpr (NORM) xv = in ? weigh(xv, wv[sp]) : zero_chunk();
-#pragma unroll
-      for (int j = 0; j < NBT; ++j)
-        if (j < nbt) acc[j] = T::mma(acc[j], in ? frag(j, sp) : zero_chunk(), xv);
-    }
-  } else {
-    const raw* xrow = static_cast<const raw*>(a.x) + static_cast<int64_t>(xr[0]) * a.x_stride;
-    u32x4 xv[SP];
-#pragma unroll
-    for (int sp = 0; sp < SP; ++sp) {
-      const int kk = kw + sp * KSTEP + g * VEC;
-      const u32x4 v = ld_chunk(xrow + (kk < a.in_dim ? kk : 0));
-      xv[sp] = kk < a.in_dim ? v : zero_chunk();
-    }
-    auto load_a = [&](int j, u32x4 (&af)[SP]) {
-      const raw* arow = a_block_row<raw>(a, en, s_first, nb_act, j < nbt ? j : 0, r16);
-#pragma unroll
-      for (int sp = 0; sp < SP; ++sp) {
-        const int kk = kw + sp * KSTEP + g * VEC;
-        af[sp] = ld_chunk(arow + (kk < a.in_dim ? kk : 0));
-      }
-    };
-    auto mma_a = [&](int j, const u32x4 (&af)[SP]) {
-#pragma unroll
-      for (int sp = 0; sp < SP; ++sp) {
-        const int kk = kw + sp * KSTEP + g * VEC;
-        acc[j] = T::mma(acc[j], kk < a.in_dim ? af[sp] : zero_chunk(), xv[sp]);
-      }
-    };
-    if constexpr (FORM == Form::kDirect) {
-      u32x4 af[NBT][SP];
-#pragma unroll
-      for (int j = 0; j < NBT; ++j) load_a(j, af[j]);
-      u32x4 wv[SP];
-      if constexpr (NORM) load_w(wv);
-      fence_regs(af);
-      if constexpr (NORM) {
-#pragma unroll
-        for (int sp = 0; sp < SP; ++sp)
-          xv[sp] = kw + sp * KSTEP + g * VEC < a.in_dim ? weigh(xv[sp], wv[sp]) : zero_chunk();
-      }
-#pragma unroll
-      for (int j = 0; j < NBT; ++j)
-        if (j < nbt) mma_a(j, af[j]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < NBT; ++j) {
-        if (j >= nbt) break;
-        u32x4 af[SP];
-        load_a(j, af);
-        mma_a(j, af);
-      }
+      u32x4 af[SP];
+      load_a(j, af);
+      mma_a(j, af, xv);
     }
   }
   MLORA_STAMP_AFTER_LOADS(2);
   if (wave > 0) {
 #pragma unroll
     for (int j = 0; j < NBT; ++j)
-      if (j < nbt) red(wave)[j * kWave + lane] = acc[j];
+      if (j < nbt) red[((wave - 1) * NBT + j) * kWave + lane] = acc[j];
   }
   lds_barrier();
   MLORA_STAMP(3);
   if (wave == 0) {
 #pragma unroll 1
-    for (int w2 = 1; w2 < 4; ++w2)
+    for (int w2 = 0; w2 < 3; ++w2)
 #pragma unroll
       for (int j = 0; j < NBT; ++j)
-        if (j < nbt) acc[j] += red(w2)[j * kWave + lane];
+        if (j < nbt) acc[j] += red[(w2 * NBT + j) * kWave + lane];
     // Lane l holds token row l & 15 and rank columns 4 (l >> 4) .. + 3 of
     // each 16-column block.
     if (r16 < en.nr) {
@@ -462,7 +398,7 @@ struct ExpandRows {
 // NORM (expand half of the fused RMSNorm launch): y = round(rstd * sum),
 // with the rstd of the thread's row t / 16 (table row yrow_raw) requested
 // with B and the output rows.
-template <class T, int NBT, int SP, int WN, int RS, bool LINKED, bool NORM = false>
+template <class T, int NBT, int SP, int WN, int RS, bool LINKED, bool NORM, bool ROWB>
 __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, const Entry& en, int nt_g,
                              const int (&orow_raw)[ExpandRows<T, WN>::RPT], DecodeLds<T, WN>& lds,
                              const float* rstd = nullptr, int yrow_raw = 0) {
@@ -501,16 +437,15 @@ __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, co
   const raw* B = static_cast<const raw*>(a.slices[s].b) + static_cast<int64_t>(en.slot) * a.slices[s].b_slot_stride;
   u32x4 bf[RS][NBW];
   u32x4 ov[RPT];
-  // Two K-steps (r_max over 32) in the two-launch schedule: eight neighbouring
-  // lanes take a B row's chunks, as in shrink_chunk, and the fragments are
-  // formed through LDS once y is ready (instruction i holds columns 8 i ..
-  // 8 i + 7 of the wave's 64).  The expand half of gate|up for 77 rows, 40
-  // entries, r_max 64: 32.1 -> 30.0 us (B's padded rows, 147 MB, at 5 TB/s).
-  // The single launch, where a workgroup's latency counts, keeps the direct
-  // loads (a 203-row prompt: 8.5 against 8.7 us).
-  constexpr bool kRowOrder = RS == 2 && !LINKED;
+  // ROWB (two K-steps, large two-launch grids; orders_of): eight neighbouring
+  // lanes take a B row's 128 bytes, and the fragments are formed through LDS
+  // once y is ready (instruction i holds columns 8 i .. 8 i + 7 of the wave's
+  // 64).  Loads in fragment order (lane l on row l % 16) ask for four cache lines
+  // every four lanes, and the CU's vector memory path then moves 38 GB/s instead
+  // of 122-128.
+  static_assert(!ROWB || (RS == 2 && !LINKED), "128-byte rows, two launches");
   auto load_b = [&]() {
-    if constexpr (kRowOrder) {
+    if constexpr (ROWB) {
       const int kk = (lane & 7) * VEC;
 #pragma unroll
       for (int i = 0; i < RS * NBW; ++i) {
@@ -591,16 +526,14 @@ __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, co
     if (miss != 0) {
       // Compute the missing chunks here, bit for bit as their shrink items
       // would, and publish them for the entry's other expand items.
-      const int xr[2] = {clamp_row(load_entry_row(plan, e, r16), a.rows), 0};
+      const int xrow = clamp_row(load_entry_row(plan, e, r16), a.rows);
       if (tid == 0) atomicAdd(a.header + kWsFallbacks, __popcll(miss));
       // The waves' sums pass through `part`, which the gather below fills.
       static_assert(3 * NBT * sizeof(f32x4[kWave]) <= sizeof(lds.part), "the sums of three waves fit");
-      f32x4* red0 = &lds.part[0][0][0];
       while (miss != 0) {
         const int z = __builtin_ctzll(miss);
         miss &= miss - 1;
-        shrink_chunk<T, NBT, SP, Form::kLean>(a, e, en, xr, sg, z, [&](int w) { return red0 + (w - 1) * NBT * kWave; }, want,
-                                        nullptr);
+        shrink_chunk<T, NBT, SP, true, false>(a, e, en, xrow, sg, z, &lds.part[0][0][0], want, nullptr);
       }
       // The prefetched B fragments and output rows are requested again, so
       // they hold no registers across the computation above (a rare path).
@@ -639,7 +572,7 @@ __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, co
   f32x4 acc[NBW];
 #pragma unroll
   for (int nb = 0; nb < NBW; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (kRowOrder) {
+  if constexpr (ROWB) {
     // Two 16-column blocks (4 KB) at a time through the wave's quarter of
     // `part`, which the barrier above has freed.
     static_assert(sizeof(lds.part) >= 4 * 4096 && NBW % 2 == 0, "4 KB a wave");
@@ -715,16 +648,11 @@ __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, co
 }
 
 // Shrink items of entries j, j + e_grid, ... (item: K chunk, and slice group
-// when the slices' A blocks are split over items).  en / xr_raw: entry j
-// and this thread's two row words (shrink_row_of), already requested.
-template <Form FORM>
-__device__ __forceinline__ int shrink_row_of(int tid, int i) {
-  return FORM == Form::kStaged ? ((tid & 63) >> 3) + 8 * i : tid & 15;
-}
-
-template <class T, int NBT, int SCHED, Form FORM, bool NORM = false>
+// when the slices' A blocks are split over items).  en / xrow_raw: entry j
+// and this thread's row word, already requested.
+template <class T, int NBT, int SCHED, bool NORM>
 __device__ void shrink_items(const int32_t* plan, const DecodeArgs& a, int j, int item, int n_ent, Entry en,
-                             int xr0_raw, int xr1_raw, unsigned char* stage, const typename T::raw_t* nw = nullptr) {
+                             int xrow_raw, f32x4* red, const typename T::raw_t* nw) {
   constexpr int SP = kGroupStepsLinked;
   int sg = 0, c = item;
   if (a.s_groups != 1) {
@@ -732,25 +660,18 @@ __device__ void shrink_items(const int32_t* plan, const DecodeArgs& a, int j, in
     c = item - sg * a.kc;
   }
   const uint64_t flag = SCHED == kGroupLinked ? flag_word() : 0;
-  // A wave's sums go where its rows were staged.
-  constexpr int kRedBytes = FORM == Form::kStaged ? kStageBytes<NBT, SP> : static_cast<int>(NBT * sizeof(f32x4[kWave]));
-  static_assert(NBT * sizeof(f32x4[kWave]) <= kRedBytes, "a wave's sums fit");
-  auto red = [&](int w) { return reinterpret_cast<f32x4*>(stage + w * kRedBytes); };
   // The first entry is taken apart from the loop over the others (rare: a
   // grid smaller than the plan), so nothing the loop hoists runs before it.
   MLORA_STAMP(1);
-  if (en.rank > 0 && en.nr > 0 && en.pos >= 0 && en.pos + en.nr <= a.ws_rows) {
-    const int xr[2] = {clamp_row(xr0_raw, a.rows), clamp_row(xr1_raw, a.rows)};
-    shrink_chunk<T, NBT, SP, FORM, NORM>(a, j, en, xr, sg, c, red, flag, stage, nw);
-  } else if (en.rank > 0 && en.nr > 0 && threadIdx.x == 0 && item == 0) {
+  if (en.rank > 0 && en.nr > 0 && en.pos >= 0 && en.pos + en.nr <= a.ws_rows)
+    shrink_chunk<T, NBT, SP, false, NORM>(a, j, en, clamp_row(xrow_raw, a.rows), sg, c, red, flag, nw);
+  else if (en.rank > 0 && en.nr > 0 && threadIdx.x == 0 && item == 0)
     atomicAdd(a.header + kWsPlanErrors, 1);
-  }
   for (int e = j + a.e_grid; e < n_ent; e += a.e_grid) {
-    const int xr[2] = {clamp_row(load_entry_row(plan, e, shrink_row_of<FORM>(threadIdx.x, 0)), a.rows),
-                       clamp_row(load_entry_row(plan, e, shrink_row_of<FORM>(threadIdx.x, 1)), a.rows)};
+    xrow_raw = load_entry_row(plan, e, threadIdx.x & 15);
     en = load_entry(plan, e, a.r_max, a.num_slots);
     if (en.rank > 0 && en.nr > 0 && en.pos >= 0 && en.pos + en.nr <= a.ws_rows)
-      shrink_chunk<T, NBT, SP, FORM, NORM>(a, e, en, xr, sg, c, red, flag, stage, nw);
+      shrink_chunk<T, NBT, SP, false, NORM>(a, e, en, clamp_row(xrow_raw, a.rows), sg, c, red, flag, nw);
     else if (en.rank > 0 && en.nr > 0 && threadIdx.x == 0 && item == 0)
       atomicAdd(a.header + kWsPlanErrors, 1);
   }
@@ -761,7 +682,7 @@ __device__ void shrink_items(const int32_t* plan, const DecodeArgs& a, int j, in
 // it cannot take.
 // NORM: rstd holds each table row's rstd; yrow_raw is the row word of entry
 // j's row threadIdx.x / 16.
-template <class T, int NBT, int WN, int RS, int SCHED, bool NORM = false>
+template <class T, int NBT, int WN, int RS, int SCHED, bool NORM, bool ROWB>
 __device__ void expand_items(const int32_t* plan, const DecodeArgs& a, int j, int tile, int n_ent, Entry en,
                              int (&rows_raw)[ExpandRows<T, WN>::RPT], DecodeLds<T, WN>& lds, bool count_errors,
                              const float* rstd = nullptr, int yrow_raw = 0) {
@@ -770,7 +691,7 @@ __device__ void expand_items(const int32_t* plan, const DecodeArgs& a, int j, in
   for (int e = j;;) {
     MLORA_STAMP(1);
     if (en.rank > 0 && en.nr > 0 && en.pos >= 0 && en.pos + en.nr <= a.ws_rows)
-      expand_entry<T, NBT, SP, WN, RS, SCHED == kGroupLinked, NORM>(a, plan, e, en, tile, rows_raw, lds, rstd,
+      expand_entry<T, NBT, SP, WN, RS, SCHED == kGroupLinked, NORM, ROWB>(a, plan, e, en, tile, rows_raw, lds, rstd,
                                                                       yrow_raw);
     else if (count_errors && en.rank > 0 && en.nr > 0 && threadIdx.x == 0 && tile == 0)
       atomicAdd(a.header + kWsPlanErrors, 1);
@@ -783,11 +704,11 @@ __device__ void expand_items(const int32_t* plan, const DecodeArgs& a, int j, in
   }
 }
 
-// Three workgroups a CU for the single launch over four A blocks (r_max 48
-// and 64): at four, the loop invariants of its expand items (their row
-// words and pointers) spilled 12-20 bytes a lane to scratch; at three it
-// holds them in 135-138 VGPRs (rank 64: 14.07 vs 13.88 us, rank 48: 11.58
-// vs 11.62 us).
+// Bound of three workgroups a CU for the single launch over four A blocks
+// (r_max 48 and 64): the compiler then stays at four with 36 bytes a lane of
+// scratch and is the fastest of what was measured (240 calls of r_max 16 to
+// 64, time against the form that held every block's fragments: 0.949; bound
+// four, no scratch, 0.965; exactly three, no scratch, 0.998).
 //
 // Workgroup (j, item) of the grid (e_grid x items) is item `item` of entry
 // j, then of entries j + e_grid, ... while the plan has them; items [0,
@@ -797,27 +718,24 @@ __device__ void expand_items(const int32_t* plan, const DecodeArgs& a, int j, in
 // as leading arguments (preloaded in SGPRs), so the first entry, the row
 // words and the plan's entry count are requested at once, together with
 // every cache line of the other arguments.
-template <class T, int NBT, int WN, int RS, int SCHED>
-__global__ __launch_bounds__(256, NBT >= 8 ? 2 : (NBT >= 4 && SCHED == kGroupLinked && RS == 2) ? 3 : 4) void planned_kernel(const int32_t* __restrict__ plan,
-                                                                       int plan_cap, int n_shrink, DecodeArgs a) {
+template <class T, int NBT, int WN, int RS, int SCHED, bool ITEM_FAST, bool ROWB>
+__global__ __launch_bounds__(256, (NBT >= 4 && SCHED == kGroupLinked && RS == 2) ? 3 : 4) void planned_kernel(
+    const int32_t* __restrict__ plan, int plan_cap, int n_shrink, DecodeArgs a) {
+  static_assert(!ITEM_FAST || SCHED != kGroupLinked, "the single launch keeps an entry on one XCD");
   // A workgroup is one kind of item: their LDS is one area.
-  constexpr Form FORM = SCHED != kGroupLinked || (NBT == 4 && RS == 2) ? Form::kStaged : Form::kDirect;
-  constexpr int kWaveLds = FORM == Form::kStaged ? kStageBytes<NBT, kGroupStepsLinked> : NBT * kWave * 16;
-  constexpr int kStage = SCHED != kGroupExpandOnly ? 4 * kWaveLds : 0;
+  constexpr int kSums = SCHED != kGroupExpandOnly ? static_cast<int>(3 * NBT * sizeof(f32x4[kWave])) : 0;
   constexpr int kExpand = SCHED != kGroupShrinkOnly ? static_cast<int>(sizeof(DecodeLds<T, WN>)) : 0;
-  __shared__ __attribute__((aligned(1024))) unsigned char area[kStage > kExpand ? kStage : kExpand];
+  __shared__ __attribute__((aligned(16))) unsigned char area[kSums > kExpand ? kSums : kExpand];
   MLORA_STAMP_BEGIN();
   constexpr int RPT = ExpandRows<T, WN>::RPT;
-  static_assert(RPT >= 2, "two row words a thread for the shrink items");
-  const bool item_fast = SCHED != kGroupLinked && a.item_fast != 0;
-  const int j = item_fast ? blockIdx.y : blockIdx.x;
-  const int item = item_fast ? blockIdx.x : blockIdx.y;
+  const int j = ITEM_FAST ? blockIdx.y : blockIdx.x;
+  const int item = ITEM_FAST ? blockIdx.x : blockIdx.y;
   const bool shrink = item < n_shrink;
   const int ef = min(j, plan_cap - 1);
   int rows_raw[RPT];
 #pragma unroll
   for (int i = 0; i < RPT; ++i)
-    rows_raw[i] = load_entry_row(plan, ef, shrink ? shrink_row_of<FORM>(threadIdx.x, i & 1) : ExpandRows<T, WN>::row_of(threadIdx.x, i));
+    rows_raw[i] = load_entry_row(plan, ef, shrink ? (threadIdx.x & 15) : ExpandRows<T, WN>::row_of(threadIdx.x, i));
   const Entry en = load_entry(plan, ef, a.r_max, a.num_slots);
   const int p0 = plan[0];
   {
@@ -835,94 +753,95 @@ __global__ __launch_bounds__(256, NBT >= 8 ? 2 : (NBT >= 4 && SCHED == kGroupLin
   if (j == 0 && item == 0 && threadIdx.x == 0 && p0 > min(plan_cap, a.e_cap)) atomicAdd(a.header + kWsPlanErrors, 1);
   if (j < n_ent) {
     if (shrink) {
-      if constexpr (SCHED != kGroupExpandOnly) shrink_items<T, NBT, SCHED, FORM>(plan, a, j, item, n_ent, en, rows_raw[0], rows_raw[1], area);
+      if constexpr (SCHED != kGroupExpandOnly)
+        shrink_items<T, NBT, SCHED, false>(plan, a, j, item, n_ent, en, rows_raw[0], reinterpret_cast<f32x4*>(area), nullptr);
     } else if constexpr (SCHED != kGroupShrinkOnly) {
-      expand_items<T, NBT, WN, RS, SCHED>(plan, a, j, item - n_shrink, n_ent, en, rows_raw,
+      expand_items<T, NBT, WN, RS, SCHED, false, ROWB>(plan, a, j, item - n_shrink, n_ent, en, rows_raw,
                                           *reinterpret_cast<DecodeLds<T, WN>*>(area), n_shrink == 0);
     }
   }
   MLORA_STAMP_FLUSH();
 }
 
-dim3 grid_of(const DecodeArgs& a, int64_t n_items, bool item_fast) {
-  const unsigned e = static_cast<unsigned>(a.e_grid), i = static_cast<unsigned>(n_items);
-  return item_fast ? dim3(i, e) : dim3(e, i);
-}
+// Instances of the two launches of a call.
+struct Orders {
+  bool shrink_fast, expand_fast;  // grid order: an entry's items next to each other (x), else the entries
+  bool row_b;                     // B rows through LDS in the expand (r_max over 32)
+};
 
-template <class T, int NBT, int WN, int RS>
-hipError_t launch_sched(const int32_t* plan, const DecodeArgs& a, int sched, int n_items, hipStream_t stream) {
+// One launch of n_items items an entry.
+template <class T, int NBT, int WN, int RS, int SCHED, bool ITEM_FAST, bool ROWB>
+hipError_t launch_sched(const int32_t* plan, const DecodeArgs& a, int n_items, hipStream_t stream) {
   if (n_items <= 0 || a.e_grid <= 0) return hipSuccess;
   if (n_items > 65535 || !grid_fits(static_cast<int64_t>(n_items) * a.e_grid)) return hipErrorInvalidConfiguration;
-  const dim3 grid = grid_of(a, n_items, sched != kGroupLinked && a.item_fast != 0);
-  const int n_shrink = sched == kGroupExpandOnly ? 0 : a.s_groups * a.kc;
-  switch (sched) {
-    case kGroupLinked:
-      hipLaunchKernelGGL((planned_kernel<T, NBT, WN, RS, kGroupLinked>), grid, dim3(256), 0, stream, plan, a.plan_cap,
-                         n_shrink, a);
-      break;
-    case kGroupShrinkOnly:
-      hipLaunchKernelGGL((planned_kernel<T, NBT, WN, RS, kGroupShrinkOnly>), grid, dim3(256), 0, stream, plan,
-                         a.plan_cap, n_shrink, a);
-      break;
-    default:
-      hipLaunchKernelGGL((planned_kernel<T, NBT, WN, RS, kGroupExpandOnly>), grid, dim3(256), 0, stream, plan,
-                         a.plan_cap, n_shrink, a);
-      break;
-  }
+  const unsigned e = static_cast<unsigned>(a.e_grid), i = static_cast<unsigned>(n_items);
+  const int n_shrink = SCHED == kGroupExpandOnly ? 0 : a.s_groups * a.kc;
+  hipLaunchKernelGGL((planned_kernel<T, NBT, WN, RS, SCHED, ITEM_FAST, ROWB>), ITEM_FAST ? dim3(i, e) : dim3(e, i),
+                     dim3(256), 0, stream, plan, a.plan_cap, n_shrink, a);
   return hipGetLastError();
 }
 
 template <class T, int NBT, int WN, int RS>
-hipError_t launch_t(const int32_t* plan, const DecodeArgs& a, int mode, int phases, hipStream_t stream) {
+hipError_t launch_t(const int32_t* plan, const DecodeArgs& a, const Orders& ord, int mode, int phases,
+                    hipStream_t stream) {
   const int n_shrink = a.s_groups * a.kc;
-  if (mode == kGroupLinked) return launch_sched<T, NBT, WN, RS>(plan, a, kGroupLinked, n_shrink + a.n_tiles, stream);
+  if (mode == kGroupLinked)
+    return launch_sched<T, NBT, WN, RS, kGroupLinked, false, false>(plan, a, n_shrink + a.n_tiles, stream);
   // Two launches: the shrink grid holds the shrink items, the expand grid
-  // the expand items (item i of entry j is workgroup i * e_grid + j there).
+  // the expand items (whose code does not depend on the A blocks).
   if (phases & 1) {
-    const hipError_t e = launch_sched<T, NBT, WN, RS>(plan, a, kGroupShrinkOnly, n_shrink, stream);
+    const hipError_t e = ord.shrink_fast
+                             ? launch_sched<T, NBT, WN, RS, kGroupShrinkOnly, true, false>(plan, a, n_shrink, stream)
+                             : launch_sched<T, NBT, WN, RS, kGroupShrinkOnly, false, false>(plan, a, n_shrink, stream);
     if (e != hipSuccess) return e;
   }
-  if (phases & 2) return launch_sched<T, NBT, WN, RS>(plan, a, kGroupExpandOnly, a.n_tiles, stream);
+  if (phases & 2) {
+    if constexpr (RS == 2) {
+      if (ord.row_b)
+        return ord.expand_fast ? launch_sched<T, 1, WN, RS, kGroupExpandOnly, true, true>(plan, a, a.n_tiles, stream)
+                               : launch_sched<T, 1, WN, RS, kGroupExpandOnly, false, true>(plan, a, a.n_tiles, stream);
+    }
+    return ord.expand_fast ? launch_sched<T, 1, WN, RS, kGroupExpandOnly, true, false>(plan, a, a.n_tiles, stream)
+                           : launch_sched<T, 1, WN, RS, kGroupExpandOnly, false, false>(plan, a, a.n_tiles, stream);
+  }
   return hipSuccess;
 }
 
 template <class T, int WN, int RS>
-hipError_t launch_nbt(const int32_t* plan, const DecodeArgs& a, int nbt, int mode, int phases, hipStream_t stream) {
+hipError_t launch_nbt(const int32_t* plan, const DecodeArgs& a, const Orders& ord, int nbt, int mode, int phases,
+                      hipStream_t stream) {
   switch (nbt) {
-    case 1: return launch_t<T, 1, WN, RS>(plan, a, mode, phases, stream);
-    case 2: return launch_t<T, 2, WN, RS>(plan, a, mode, phases, stream);
-    default: return launch_t<T, 4, WN, RS>(plan, a, mode, phases, stream);
+    case 1: return launch_t<T, 1, WN, RS>(plan, a, ord, mode, phases, stream);
+    case 2: return launch_t<T, 2, WN, RS>(plan, a, ord, mode, phases, stream);
+    default: return launch_t<T, 4, WN, RS>(plan, a, ord, mode, phases, stream);
   }
 }
 
 template <class T>
-hipError_t launch_dtype(const int32_t* plan, const DecodeArgs& a, int nbt, int mode, int phases, hipStream_t stream) {
-  if (a.r_max <= T::KSTEP) return launch_nbt<T, 1, 1>(plan, a, nbt, mode, phases, stream);
-  return launch_nbt<T, 1, 2>(plan, a, nbt, mode, phases, stream);
+hipError_t launch_dtype(const int32_t* plan, const DecodeArgs& a, const Orders& ord, int nbt, int mode, int phases,
+                        hipStream_t stream) {
+  if (a.r_max <= T::KSTEP) return launch_nbt<T, 1, 1>(plan, a, ord, nbt, mode, phases, stream);
+  return launch_nbt<T, 1, 2>(plan, a, ord, nbt, mode, phases, stream);
 }
 
 // ------------------------------------------- fused RMSNorm + decode shrink
-// Shrink launch: grid (e_grid, norm rows + n_shrink).  Workgroup (j, i)
-// for i < n_norm is RMSNorm row block i * e_grid + j (256 / tpr rows),
-// written as the RMSNorm kernel writes it, with each row's rstd stored; the
+// Shrink launch: grid (e_grid, norm rows + n_shrink), or with ITEM_FAST
+// (n_shrink, norm rows + e_grid).  The first n_norm rows of the grid are
+// RMSNorm row blocks in turn (256 / tpr rows each), written as the RMSNorm kernel writes it, with each row's rstd stored; the
 // items after them are the shrink items of the two-launch schedule, with
 // round(x * w) on the MFMA.  The norm rows come first in the grid, so they
 // run beside the first shrink items instead of after the last.  Nothing in
 // the launch waits on another workgroup.
-template <class T, int NBT, Form FORM>
+template <class T, int NBT, bool ITEM_FAST>
 __global__ __launch_bounds__(256, 4) void planned_norm_shrink_kernel(const int32_t* __restrict__ plan,
                                                                                      int plan_cap, int n_norm,
                                                                                      DecodeArgs a, NormShrinkArgs na) {
-  // The norm rows' four words lie in the area the shrink items stage in (at
-  // four A blocks it is a quarter of a CU's LDS, and one word more would cost
-  // a workgroup).
-  constexpr int kWaveLds = FORM == Form::kStaged ? kStageBytes<NBT, kGroupStepsLinked> : NBT * kWave * 16;
-  __shared__ __attribute__((aligned(1024))) unsigned char stage[4 * kWaveLds];
-  float* nred = reinterpret_cast<float*>(stage);
+  __shared__ f32x4 red[3 * NBT * kWave];
+  __shared__ float nred[4];
   // Rows [0, n_norm) of the grid are the norm row blocks.
   const int y = static_cast<int>(blockIdx.y) - n_norm;
-  const int item = a.item_fast ? static_cast<int>(blockIdx.x) : y;
-  const int j = a.item_fast ? y : static_cast<int>(blockIdx.x);
+  const int item = ITEM_FAST ? static_cast<int>(blockIdx.x) : y;
+  const int j = ITEM_FAST ? y : static_cast<int>(blockIdx.x);
   if (y < 0) {
     const int64_t blk = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
     // At most two chunks a thread held (the rest streamed twice): the same
@@ -932,8 +851,7 @@ __global__ __launch_bounds__(256, 4) void planned_norm_shrink_kernel(const int32
     return;
   }
   const int ef = min(j, plan_cap - 1);
-  const int row0_raw = load_entry_row(plan, ef, shrink_row_of<FORM>(threadIdx.x, 0));
-  const int row1_raw = load_entry_row(plan, ef, shrink_row_of<FORM>(threadIdx.x, 1));
+  const int row_raw = load_entry_row(plan, ef, threadIdx.x & 15);
   const Entry en = load_entry(plan, ef, a.r_max, a.num_slots);
   const int p0 = plan[0];
   {
@@ -949,19 +867,19 @@ __global__ __launch_bounds__(256, 4) void planned_norm_shrink_kernel(const int32
   const int n_ent = min(p0, min(plan_cap, a.e_cap));
   if (j == 0 && item == 0 && threadIdx.x == 0 && p0 > min(plan_cap, a.e_cap)) atomicAdd(a.header + kWsPlanErrors, 1);
   if (j < n_ent)
-    shrink_items<T, NBT, kGroupShrinkOnly, FORM, true>(plan, a, j, item, n_ent, en, row0_raw, row1_raw, stage,
+    shrink_items<T, NBT, kGroupShrinkOnly, true>(plan, a, j, item, n_ent, en, row_raw, red,
                                                  static_cast<const typename T::raw_t*>(na.rms.w));
 }
 
 // Expand launch: the expand items of the two-launch schedule, y scaled by
 // each row's rstd before its rounding.
-template <class T, int WN, int RS>
+template <class T, int WN, int RS, bool ITEM_FAST, bool ROWB>
 __global__ __launch_bounds__(256, 4) void planned_norm_expand_kernel(const int32_t* __restrict__ plan, int plan_cap,
                                                                      DecodeArgs a, const float* __restrict__ rstd) {
   __shared__ __attribute__((aligned(16))) DecodeLds<T, WN> lds;
   constexpr int RPT = ExpandRows<T, WN>::RPT;
-  const int j = a.item_fast ? blockIdx.y : blockIdx.x;
-  const int item = a.item_fast ? blockIdx.x : blockIdx.y;
+  const int j = ITEM_FAST ? blockIdx.y : blockIdx.x;
+  const int item = ITEM_FAST ? blockIdx.x : blockIdx.y;
   const int ef = min(j, plan_cap - 1);
   int rows_raw[RPT];
 #pragma unroll
@@ -983,60 +901,74 @@ __global__ __launch_bounds__(256, 4) void planned_norm_expand_kernel(const int32
   if (j == 0 && item == 0 && threadIdx.x == 0 && p0 > min(plan_cap, a.e_cap))
     atomicAdd(a.header + kWsPlanErrors, 1);
   if (j < n_ent)
-    expand_items<T, 1, WN, RS, kGroupExpandOnly, true>(plan, a, j, item, n_ent, en, rows_raw, lds, true,
-                                                           rstd, yrow_raw);
+    expand_items<T, 1, WN, RS, kGroupExpandOnly, true, ROWB>(plan, a, j, item, n_ent, en, rows_raw, lds, true, rstd,
+                                                             yrow_raw);
+}
+
+// Rows of the norm + shrink grid: norm row blocks, then entries (ITEM_FAST) or
+// shrink items.
+struct NormGrid {
+  int64_t per_row, n_norm, rows;
+};
+NormGrid norm_grid(const DecodeArgs& a, const NormShrinkArgs& na, bool item_fast) {
+  const int64_t n_shrink = static_cast<int64_t>(a.s_groups) * a.kc;
+  const int64_t blocks = (na.rms.rows + (256 / na.rms.tpr) - 1) / (256 / na.rms.tpr);
+  NormGrid g;
+  g.per_row = item_fast ? n_shrink : a.e_grid;
+  g.n_norm = (blocks + g.per_row - 1) / g.per_row;
+  g.rows = g.n_norm + (item_fast ? a.e_grid : n_shrink);
+  return g;
+}
+
+template <class T, int NBT, bool ITEM_FAST>
+hipError_t launch_norm_shrink(const int32_t* plan, const DecodeArgs& a, const NormShrinkArgs& na, hipStream_t stream) {
+  if (a.e_grid <= 0 || na.rms.rows <= 0) return hipSuccess;
+  const NormGrid g = norm_grid(a, na, ITEM_FAST);
+  if (g.rows > 65535 || !grid_fits(g.rows * g.per_row)) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, ITEM_FAST>),
+                     dim3(static_cast<unsigned>(g.per_row), static_cast<unsigned>(g.rows)), dim3(256), 0, stream, plan,
+                     a.plan_cap, static_cast<int>(g.n_norm), a, na);
+  return hipGetLastError();
 }
 
 template <class T, int NBT>
-hipError_t launch_norm_shrink(const int32_t* plan, const DecodeArgs& a, const NormShrinkArgs& na, hipStream_t stream) {
-  const int n_shrink = a.s_groups * a.kc;
-  if (a.e_grid <= 0 || na.rms.rows <= 0) return hipSuccess;
-  const int64_t blocks = (na.rms.rows + (256 / na.rms.tpr) - 1) / (256 / na.rms.tpr);
-  const int64_t per_row = a.item_fast ? n_shrink : a.e_grid;
-  const int64_t n_norm = (blocks + per_row - 1) / per_row;
-  const int64_t grid_y = n_norm + (a.item_fast ? a.e_grid : n_shrink);
-  if (grid_y > 65535 || !grid_fits(grid_y * per_row)) return hipErrorInvalidConfiguration;
-  const dim3 grid(static_cast<unsigned>(per_row), static_cast<unsigned>(grid_y));
-  // Direct loads for a grid of at most four workgroups a CU, which runs at once
-  // and is bound by one workgroup's latency (a layer of 14 rows over one
-  // adapter: 37.5 against 38.2 us), and for items of one or two A blocks: the
-  // norm rows share the launch, and the LDS that staging takes (24 KB a
-  // workgroup) keeps waves off the CU that direct loads let run (q|k|v of 256
-  // rows, 112 rank-32 adapters, the whole call: 39.1 against 40.7 us staged).
-  if constexpr (NBT > 2) {
-    if (a.item_fast) {
-      hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kStaged>), grid, dim3(256), 0, stream, plan,
-                         a.plan_cap, static_cast<int>(n_norm), a, na);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((planned_norm_shrink_kernel<T, NBT, Form::kDirect>), grid, dim3(256), 0, stream, plan, a.plan_cap,
-                     static_cast<int>(n_norm), a, na);
+hipError_t launch_norm_shrink_order(const int32_t* plan, const DecodeArgs& a, const Orders& ord,
+                                    const NormShrinkArgs& na, hipStream_t stream) {
+  return ord.shrink_fast ? launch_norm_shrink<T, NBT, true>(plan, a, na, stream)
+                         : launch_norm_shrink<T, NBT, false>(plan, a, na, stream);
+}
+
+template <class T, int RS, bool ITEM_FAST, bool ROWB>
+hipError_t launch_norm_expand(const int32_t* plan, const DecodeArgs& a, const float* rstd, hipStream_t stream) {
+  if (a.e_grid <= 0 || a.n_tiles <= 0) return hipSuccess;
+  if (a.n_tiles > 65535 || !grid_fits(static_cast<int64_t>(a.n_tiles) * a.e_grid)) return hipErrorInvalidConfiguration;
+  const unsigned e = static_cast<unsigned>(a.e_grid), i = static_cast<unsigned>(a.n_tiles);
+  hipLaunchKernelGGL((planned_norm_expand_kernel<T, 1, RS, ITEM_FAST, ROWB>), ITEM_FAST ? dim3(i, e) : dim3(e, i),
+                     dim3(256), 0, stream, plan, a.plan_cap, a, rstd);
   return hipGetLastError();
 }
 
 template <class T>
-hipError_t launch_norm_t(const int32_t* plan, const DecodeArgs& a, const NormShrinkArgs& na, int nbt, int phases,
+hipError_t launch_norm_t(const int32_t* plan, const DecodeArgs& a, const Orders& ord, const NormShrinkArgs& na, int nbt, int phases,
                          hipStream_t stream) {
   if (phases & 1) {
     hipError_t e;
     switch (nbt) {
-      case 1: e = launch_norm_shrink<T, 1>(plan, a, na, stream); break;
-      case 2: e = launch_norm_shrink<T, 2>(plan, a, na, stream); break;
-      default: e = launch_norm_shrink<T, 4>(plan, a, na, stream); break;
+      case 1: e = launch_norm_shrink_order<T, 1>(plan, a, ord, na, stream); break;
+      case 2: e = launch_norm_shrink_order<T, 2>(plan, a, ord, na, stream); break;
+      default: e = launch_norm_shrink_order<T, 4>(plan, a, ord, na, stream); break;
     }
     if (e != hipSuccess) return e;
   }
-  if ((phases & 2) && a.e_grid > 0 && a.n_tiles > 0) {
-    if (a.n_tiles > 65535 || !grid_fits(static_cast<int64_t>(a.n_tiles) * a.e_grid)) return hipErrorInvalidConfiguration;
-    const dim3 grid = grid_of(a, a.n_tiles, a.item_fast != 0);
+  if (phases & 2) {
     if (a.r_max <= T::KSTEP)
-      hipLaunchKernelGGL((planned_norm_expand_kernel<T, 1, 1>), grid, dim3(256), 0, stream, plan, a.plan_cap, a,
-                         na.rstd);
-    else
-      hipLaunchKernelGGL((planned_norm_expand_kernel<T, 1, 2>), grid, dim3(256), 0, stream, plan, a.plan_cap, a,
-                         na.rstd);
-    return hipGetLastError();
+      return ord.expand_fast ? launch_norm_expand<T, 1, true, false>(plan, a, na.rstd, stream)
+                           : launch_norm_expand<T, 1, false, false>(plan, a, na.rstd, stream);
+    if (ord.row_b)
+      return ord.expand_fast ? launch_norm_expand<T, 2, true, true>(plan, a, na.rstd, stream)
+                           : launch_norm_expand<T, 2, false, true>(plan, a, na.rstd, stream);
+    return ord.expand_fast ? launch_norm_expand<T, 2, true, false>(plan, a, na.rstd, stream)
+                         : launch_norm_expand<T, 2, false, false>(plan, a, na.rstd, stream);
   }
   return hipSuccess;
 }
@@ -1242,23 +1174,41 @@ hipError_t launch_build_plan(const SegView& m, int rows, int32_t* plan, int cap,
   return hipGetLastError();
 }
 
-static DecodeArgs with_grid_order(DecodeArgs a) {
-  a.item_fast = static_cast<int64_t>(a.e_grid) * a.s_groups * a.kc > kDirectItems && a.e_grid <= 32768;
-  return a;
+// Which instances a call's two launches run (us, start of the line / with it):
+//   shrink, an entry's items next to each other, past kDirectBlocks A blocks
+//     of items: q|k|v of 256 rows over 112 adapters at rank 32 23.6 / 20.3, at
+//     rank 64 38.1 / 36.2; down of 128 rows over 128 adapters at rank 64 57.8 /
+//     48.0.  Smaller grids keep an entry on one XCD (1.00-1.03 of their time
+//     otherwise).
+//   expand, the same order, from 56 column tiles or 40 in a grid of 2048 items,
+//     r_max over 16: gate|up of 77 rows over 40 adapters in r_max 64 36.2 / 33.6;
+//     narrower outputs 1.02-1.2 of their time, r_max 16 the same either way.
+//   expand, B in row order through LDS, past 2048 items at r_max over 32: the same
+//     gate|up 33.6 / 31.5, q|k|v of 128 rows over 128 adapters 24.5 / 23.5;
+//     smaller grids 1.00-1.06 of their time.
+static Orders orders_of(const DecodeArgs& a, int nbt) {
+  const int64_t shrink_items = static_cast<int64_t>(a.e_grid) * a.s_groups * a.kc;
+  const int64_t expand_items = static_cast<int64_t>(a.e_grid) * a.n_tiles;
+  const bool y_fits = a.e_grid <= 65535;  // entries along y
+  Orders o;
+  o.shrink_fast = y_fits && shrink_items * nbt > kDirectBlocks;
+  o.expand_fast = y_fits && a.r_max > 16 && (a.n_tiles >= 56 || (a.n_tiles >= 40 && expand_items > 2048));
+  o.row_b = a.r_max > 32 && expand_items > 2048;
+  return o;
 }
 
-hipError_t launch_planned(const int32_t* plan, const DecodeArgs& in, int dtype, int nbt, int mode, int phases,
+hipError_t launch_planned(const int32_t* plan, const DecodeArgs& args, int dtype, int nbt, int mode, int phases,
                           hipStream_t stream) {
-  const DecodeArgs args = with_grid_order(in);
-  if (dtype == MLORA_BF16) return launch_dtype<BF16>(plan, args, nbt, mode, phases, stream);
-  return launch_dtype<F16>(plan, args, nbt, mode, phases, stream);
+  const Orders ord = orders_of(args, nbt);
+  if (dtype == MLORA_BF16) return launch_dtype<BF16>(plan, args, ord, nbt, mode, phases, stream);
+  return launch_dtype<F16>(plan, args, ord, nbt, mode, phases, stream);
 }
 
-hipError_t launch_planned_norm(const int32_t* plan, const DecodeArgs& in, const NormShrinkArgs& na, int dtype,
+hipError_t launch_planned_norm(const int32_t* plan, const DecodeArgs& args, const NormShrinkArgs& na, int dtype,
                                int nbt, int phases, hipStream_t stream) {
-  const DecodeArgs args = with_grid_order(in);
-  if (dtype == MLORA_BF16) return launch_norm_t<BF16>(plan, args, na, nbt, phases, stream);
-  return launch_norm_t<F16>(plan, args, na, nbt, phases, stream);
+  const Orders ord = orders_of(args, nbt);
+  if (dtype == MLORA_BF16) return launch_norm_t<BF16>(plan, args, ord, na, nbt, phases, stream);
+  return launch_norm_t<F16>(plan, args, ord, na, nbt, phases, stream);
 }
 
 }  // namespace mlora

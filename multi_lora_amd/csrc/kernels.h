@@ -205,7 +205,6 @@ struct DecodeArgs {
   int n_tiles;       // expand items per entry (256-column tiles over all slices)
   int tile_base[kMaxSlices + 1];
   int e_grid;        // entries the grid holds (multiple of 8)
-  int item_fast;     // grid order: an entry's items next to each other (x), else the entries
   int e_cap;         // entries the workspace flags hold
   int plan_cap;      // entries the plan holds
   int ws_rows;       // rows the workspace sums hold

@@ -879,7 +879,7 @@ hipError_t launch_dtype(const ShrinkPlan& p, const ShrinkArgs& args, int dtype, 
 // reduction (shrink_wide.hip) rather than split over workgroups.  What counts
 // is the bytes a tile reads, its 16 rows of x and every A block over all of K,
 // which one CU loads, and how full the tiles are: a one-row segment reads as
-// much as a 16-row one.  Measured on 1,360 whole calls, cold inputs, K 255 to
+// much as a 16-row one.  Measured on 1,268 whole calls, cold inputs, K 255 to
 // 14336, ranks 8 to 128, 17 to 4075 rows (time as wide / time as split, by
 // bytes a tile):
 //   16-bit, segments of 64 rows and more on average: up to 192 KB 0.69-1.01,

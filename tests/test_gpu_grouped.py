@@ -552,15 +552,19 @@ def test_largest_supported_shape(dev):
     assert counters(lws)[0] > 0
 
 
-@pytest.mark.parametrize("in_dim,out,r_max,ranks", [
-    (4104, 264, 64, [64, 33, 8, 16]),    # last K chunk of one 16-byte piece, a ragged column tile
-    (2552, 512, 40, [40, 13]),           # B rows of five pieces
-    (4096, 768, 24, [24, 8, 17]),
+@pytest.mark.parametrize("in_dim,out,r_max,ranks,n_slots", [
+    (4104, 264, 64, [64, 33, 8, 16], 130),    # last K chunk of one 16-byte piece, a ragged column tile
+    (2552, 512, 40, [40, 13], 130),           # B rows of five pieces, row order
+    (4096, 768, 24, [24, 8, 17], 130),
+    (1032, 14344, 64, [64, 16, 48], 40),      # wide: expand items next to each other, B in row order
+    (520, 14344, 32, [32, 7], 40),            # the same with one K-step of B
+    (520, 10248, 48, [33, 48], 56),           # 41 column tiles
 ])
-def test_large_two_launch_grids_equal_the_single_launch(dev, in_dim, out, r_max, ranks):
-    """Grids of more than 1024 shrink items (staged rows, an entry's items next
-    to each other) against the single launch, bit for bit, and the oracle."""
-    n_slots, rows = 130, 200
+def test_large_two_launch_grids_equal_the_single_launch(dev, in_dim, out, r_max, ranks, n_slots):
+    """Large grids of the two launches (an entry's items next to each other in
+    the shrink, the expand or both, B in row order) against the single launch,
+    bit for bit, and the oracle."""
+    rows = n_slots + 70
     g = torch.Generator().manual_seed(in_dim)
     slots = [i % n_slots for i in range(rows)]
     slot_ranks = [ranks[i % len(ranks)] for i in range(n_slots)]
@@ -570,7 +574,8 @@ def test_large_two_launch_grids_equal_the_single_launch(dev, in_dim, out, r_max,
     base = torch.randn(rows, out, generator=g).bfloat16()
     scal = [0.5 + (i % 3) for i in range(n_slots)]
     meta = make_meta([1] * rows, slots, slot_ranks, scal, dev, torch.bfloat16)
-    assert meta.plan_entries * -(-in_dim // 256) > 1024
+    shrink_blocks = meta.plan_entries * -(-in_dim // 256) * -(-r_max // 16)
+    assert shrink_blocks > 1024 or meta.plan_entries * -(-out // 256) > 2048
     outs = []
     for mode in (1, 2):
         got = base.to(dev)

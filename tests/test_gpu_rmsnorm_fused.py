@@ -103,6 +103,22 @@ def test_widths(dev, in_dim):
     check(wl, scaled(wl.x, 5), norm_weight(in_dim, wl.x.dtype, dev, 5), 1e-5, f"in {in_dim}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("in_dim,outs", [(4096, [1024, 256, 264]), (4104, [512, 256, 256]), (1032, [14344])])
+def test_large_grids_of_mixed_ranks(dev, in_dim, outs, dtype):
+    """77 rows over 40 adapters of ranks 8 to 64 in r_max 64: four A blocks an
+    item, an entry's items next to each other behind the norm row blocks, and
+    with the wide output the expand in that order too, B in row order."""
+    slots, ranks = [i % 40 for i in range(77)], [(64, 33, 8, 16)[i % 4] for i in range(40)]
+    wl = workload("mixed ranks", dev, [1] * 77, slots, ranks, [0.5 + (i % 3) for i in range(40)], in_dim, outs, 64,
+                  in_dim % 89, dtype=dtype)
+    blocks = wl.meta.plan_entries * len(outs) * -(-in_dim // 256) * 4
+    assert blocks > 1024 or wl.meta.plan_entries * -(-outs[0] // 256) > 2048
+    # fp16's x * w stays finite: rows are not scaled there.
+    x = scaled(wl.x, 11) if dtype == torch.bfloat16 else wl.x
+    check(wl, x, norm_weight(in_dim, dtype, dev, 11), 1e-5, f"mixed ranks {in_dim} {outs} {dtype}")
+
+
 def test_multi_row_segments_and_rank0(dev):
     """Segments of several rows (entries of up to 16 rows, a slot split over
     entries), rank-0 slots whose rows still get y and keep their output."""
