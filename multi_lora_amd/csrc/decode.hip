@@ -931,11 +931,13 @@ hipError_t launch_norm_shrink(const int32_t* plan, const DecodeArgs& a, const No
   return hipGetLastError();
 }
 
+// The items next to each other, unless that makes the grid too tall (its rows
+// are short, and the norm row blocks fill them first).
 template <class T, int NBT>
 hipError_t launch_norm_shrink_order(const int32_t* plan, const DecodeArgs& a, const Orders& ord,
                                     const NormShrinkArgs& na, hipStream_t stream) {
-  return ord.shrink_fast ? launch_norm_shrink<T, NBT, true>(plan, a, na, stream)
-                         : launch_norm_shrink<T, NBT, false>(plan, a, na, stream);
+  return ord.shrink_fast && norm_grid(a, na, true).rows <= 65535 ? launch_norm_shrink<T, NBT, true>(plan, a, na, stream)
+                                                                 : launch_norm_shrink<T, NBT, false>(plan, a, na, stream);
 }
 
 template <class T, int RS, bool ITEM_FAST, bool ROWB>
