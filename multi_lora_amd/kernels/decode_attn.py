@@ -20,11 +20,21 @@ from torch.utils._device import DeviceContext
 from .. import _ffi
 
 _DTYPES = (torch.float16, torch.bfloat16)
-# One workgroup takes a key head's whole cache: with fewer than 64 of them the
-# chip is nearly idle, and past 1024 positions torch's launches catch up (4
-# key heads, 2048 positions: 53.0 against 51.8 us; 64: 64.3 against 64.5; at
-# 512 key heads 166 against 204, and at 520 positions 57 against 96).
-MAX_LEN, MAX_LEN_FEW_HEADS, FEW_HEADS = 2048, 1024, 64
+# Longest cache taken.  One workgroup takes a key head's whole cache: with
+# fewer than 64 of them the chip is nearly idle, and past 1024 positions torch's
+# launches catch up (4 key heads, 2048 positions: 53.0 against 51.8 us; 64: 64.3
+# against 64.5; at 512 key heads 166 against 204, and at 520 positions 57 against
+# 96).  Eight query heads a key head fill a CU's LDS with one workgroup, and
+# torch's catch up earlier (the layer with its projections, 1 key head, 1024
+# positions: 60-62 against 52-53; 4: 79 against 75; 128 key heads, 2048 positions:
+# 114-118 against 110-111, 1024: faster).
+FEW_HEADS = 64
+
+
+def _max_len(key_heads: int, rep: int) -> int:
+    if rep == 8:
+        return 1024 if key_heads >= FEW_HEADS else 600
+    return 2048 if key_heads >= FEW_HEADS else 1024
 
 
 def _followed() -> bool:
@@ -58,15 +68,15 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
     cache, except the positions ``hide [b, 1, 1, L]`` marks; ``[b, heads*d]``.
     A ``pos`` outside the cache, which only the device knows, writes nothing
     and makes the result NaN."""
-    if not _plain(q, k, v, cos, sin, keys, values, hide, pos) or values.dim() != 4:
+    if values.dim() != 4:
         return None
     b, kv_heads, length, d = values.shape
-    if length > (MAX_LEN if b * kv_heads >= FEW_HEADS else MAX_LEN_FEW_HEADS):
-        return None
     if d not in (64, 128) or q.dim() != 2 or q.shape[1] % d or b == 0:
         return None
     heads = q.shape[1] // d
-    if heads % kv_heads or heads // kv_heads not in (1, 2, 4, 8):
+    if heads % kv_heads or heads // kv_heads not in (1, 2, 4, 8) or length > _max_len(b * kv_heads, heads // kv_heads):
+        return None
+    if not _plain(q, k, v, cos, sin, keys, values, hide, pos):
         return None
     rows = (q, k, v)
     if any(t.dtype != q.dtype for t in (k, v, cos, sin, keys, values)) or any(t.stride(1) != 1 for t in rows):

@@ -44,3 +44,9 @@ def test_transforms_tracing_and_compilation(monkeypatch):
     assert seen == [True] * 4
     monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
     assert decode_attn._followed()
+
+
+@pytest.mark.parametrize("key_heads,rep,longest", [(1, 8, 600), (63, 8, 600), (64, 8, 1024), (1, 4, 1024), (63, 1, 1024),
+                                                   (64, 4, 2048), (512, 2, 2048)])
+def test_longest_cache_by_the_workgroups_it_makes(key_heads, rep, longest):
+    assert decode_attn._max_len(key_heads, rep) == longest

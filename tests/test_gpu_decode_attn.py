@@ -197,3 +197,11 @@ def test_the_cache_write_is_counted_and_inference_caches_stay_refused(dev):
         made = inputs(dev, 2, 4, 2, 64, 40, torch.bfloat16, 0, 1)
         assert decode_attention(*made, at, 0.125) is not None
     assert decode_attention(*made, at, 0.125) is None
+
+
+@pytest.mark.parametrize("heads,length", [(8, 600), (4, 1024)])
+def test_caches_past_the_longest_one_are_left_to_torch(dev, heads, length):
+    at = torch.tensor([1], device=dev)
+    for n, taken in ((length, True), (length + 1, False)):
+        args = inputs(dev, 1, heads, 1, 64, n, torch.bfloat16, 0, 1)
+        assert (decode_attention(*args, at, 0.125) is not None) is taken
