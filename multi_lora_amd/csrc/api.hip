@@ -684,7 +684,7 @@ int mlora_decode_attention(const void* q, int64_t q_row_stride, const void* k, i
     return fail(kBadArg, "batch %d, heads %d, kv_heads %d, len %d", batch, heads, kv_heads, len);
   const int rep = heads / kv_heads;
   if ((head_dim != 64 && head_dim != 128) || (rep != 1 && rep != 2 && rep != 4 && rep != 8) || len > mlora::kAttnMaxLen ||
-      !al16(values) || static_cast<int64_t>(batch) * kv_heads > mlora::kMaxBlocks)
+      !al16(values) || !mlora::grid_fits(static_cast<int64_t>(batch) * kv_heads * (mlora::kAttnThreads / 256)))
     return fail(kUnsupported, "decode attention takes head_dim 64 or 128 (got %d), 1, 2, 4 or 8 heads a key head (%d), "
                 "caches of up to %d (%d), 16-byte aligned values", head_dim, rep, mlora::kAttnMaxLen, len);
   if (batch == 0) return 0;

@@ -30,7 +30,6 @@ namespace mlora {
 
 namespace {
 
-constexpr int kAttnThreads = 512;
 constexpr int kAttnWaves = kAttnThreads / kWave;
 constexpr int kAttnChunk = 256;  // positions a pass
 

@@ -313,6 +313,7 @@ hipError_t launch_scatter(const ScatterArgs& args, int64_t max_numel, int elem_b
 // -------------------------------------------------------------- decoder
 // Longest cache the decode attention's scores fit in LDS for.
 constexpr int kAttnMaxLen = 2048;
+constexpr int kAttnThreads = 512;
 
 struct AttnArgs {
   const void *q, *k, *v;  // rows of the new tokens [batch, heads * D]

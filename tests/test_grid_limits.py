@@ -29,3 +29,17 @@ def test_fused_norm_of_many_short_rows_is_not_too_tall_a_grid():
     rc = lib.mlora_rmsnorm_apply_grouped(1 << 43, k, rows, k, 1 << 44, 1e-5, 1 << 45, k, sl, 1, r, 1 << 46, 256,
                                          ctypes.byref(meta), _ffi.MLORA_BF16, 1 << 47, need, 1, None)
     assert rc > 0 and rc != INVALID_CONFIGURATION, lib.mlora_last_error()
+
+
+def test_decode_attention_counts_its_512_threads():
+    """More workgroups than fit a launch's 2^32 work-items are turned down
+    before anything else is looked at (null pointers here)."""
+    lib = _ffi.lib()
+
+    def call(batch):
+        return lib.mlora_decode_attention(None, 64, None, 64, None, 64, None, None, 0, None, None, None, 0, None, None,
+                                          64, batch, 1, 1, 64, 8, 0.125, _ffi.MLORA_BF16, None)
+
+    most = (2 ** 32 - 1) // 512
+    assert call(most) == -1 and b"null" in lib.mlora_last_error()
+    assert call(most + 1) == -2
