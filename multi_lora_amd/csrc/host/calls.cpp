@@ -247,6 +247,16 @@ struct Slices {
   mlora_slice s[MLORA_MAX_SLICES]{};
   int n = 0;
   int64_t r_max = 0, slots = 0, width = 0;
+  // The stacks, for the length of the call: a list may lose them while a
+  // workspace's get runs, or while the interpreter's lock is released.
+  PyObject* held[2 * MLORA_MAX_SLICES] = {};
+
+  Slices() = default;
+  Slices(const Slices&) = delete;
+  Slices& operator=(const Slices&) = delete;
+  ~Slices() {
+    for (PyObject* o : held) Py_XDECREF(o);
+  }
 
   bool read(PyObject* a, PyObject* b, PyObject* cols, const at::Tensor& x) {
     if (!is_seq(a) || !is_seq(b) || (cols != Py_None && !is_seq(cols))) return false;
@@ -257,8 +267,10 @@ struct Slices {
     slots = INT32_MAX;
     int64_t col = 0;
     for (int i = 0; i < n; ++i) {
-      const at::Tensor* ta = tensor_of(PySequence_Fast_GET_ITEM(a, i));
-      const at::Tensor* tb = tensor_of(PySequence_Fast_GET_ITEM(b, i));
+      Py_XINCREF(held[2 * i] = PySequence_Fast_GET_ITEM(a, i));
+      Py_XINCREF(held[2 * i + 1] = PySequence_Fast_GET_ITEM(b, i));
+      const at::Tensor* ta = tensor_of(held[2 * i]);
+      const at::Tensor* tb = tensor_of(held[2 * i + 1]);
       if (ta == nullptr || tb == nullptr || !is_stack(*ta, x) || !is_stack(*tb, x)) return false;
       if (i == 0) r_max = ta->size(1);
       if (ta->size(1) != r_max || tb->size(2) != r_max || ta->size(2) != x.size(1)) return false;
@@ -397,9 +409,10 @@ PyObject* sgemm_a(PyObject* const* args, Took* took) {
   size_t ws_bytes = 0;
   if (need != 0) {
     Ref key(Py_BuildValue("(OiO)", s_cuda, static_cast<int>(dev.index()), Py_False));
-    PyObject* held = key.p != nullptr ? PyDict_GetItemWithError(args[5], key.p) : nullptr;
-    if (held == nullptr) return nullptr;
-    *took = workspace(held, need, *x, args[0], &ws, &ws_bytes);
+    Ref held(key.p != nullptr ? PyDict_GetItemWithError(args[5], key.p) : nullptr);
+    if (held.p == nullptr) return nullptr;
+    Py_INCREF(held.p);  // the dict's own reference was borrowed
+    *took = workspace(held.p, need, *x, args[0], &ws, &ws_bytes);
     if (*took != Took::kYes) return nullptr;
   }
   mlora_slice s{};

@@ -111,3 +111,29 @@ def test_native_fused_norm_and_two_call_forms(dev):
     assert sgemm_lora_b_fwd(mid, p.b_stacks[0], p.meta, one) is one
     expand(mid, [p.b_stacks[0]], p.meta, two, [0])
     assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("make", [decode, prompts])
+def test_stacks_live_for_the_length_of_the_call(dev, make):
+    """A list that loses its stacks while the call makes its workspace: their
+    memory may go to other tensors only after the call."""
+    wl = make(dev)
+    want, got = wl.clone_base(), wl.clone_base()
+    assert taken(wl, want, cols=wl.col_offsets) is True
+    a, b = [t.clone() for t in wl.a_stacks], [t.clone() for t in wl.b_stacks]
+    sizes = [t.numel() for t in a + b]
+    spoilt = []
+
+    def spoil(get):
+        def run(*args):
+            a.clear()
+            b.clear()
+            spoilt.extend(torch.full((n,), float("nan"), dtype=wl.x.dtype, device=dev) for n in sizes)
+            return get(*args)
+        return run
+
+    linked, seg = LinkedWorkspace(), Workspace()
+    linked.get, seg.get = spoil(linked.get), spoil(seg.get)
+    assert taken(wl, got, a=a, b=b, cols=wl.col_offsets, linked=linked, seg=seg) is True
+    torch.cuda.synchronize()
+    assert spoilt and torch.equal(got, want)
