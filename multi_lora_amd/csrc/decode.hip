@@ -585,12 +585,14 @@ __device__ void expand_entry(const DecodeArgs& a, const int32_t* plan, int e, co
     }
 #pragma unroll
     for (int nb = 0; nb < NBW; nb += 2) {
+      wave_lds_fence();  // the last two blocks' fragments are read
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int f = nb * 2 + i;  // load instruction
         const int row = i * 8 + (lane >> 3);
         *reinterpret_cast<u32x4*>(mine + row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4)) = bf[f / NBW][f % NBW];
       }
+      wave_lds_fence();
 #pragma unroll
       for (int ks = 0; ks < RS; ++ks) {
         if (ks * KSTEP >= rank) break;

@@ -185,8 +185,10 @@ __device__ __forceinline__ void expand_dma_tile(const ExpandArgs& a, const TileR
     for (int nb = 0; nb < 4; ++nb) {
 #pragma unroll
       for (int i = 0; i < 16 / BROWS; ++i) put(mine, i * BROWS + lane / LPB, braw[nb * (16 / BROWS) + i]);
+      wave_lds_fence();
 #pragma unroll
       for (int ks = 0; ks < RS; ++ks) bf[ks][nb] = frag(mine, r16, ks) & keep_mask<T>(rank - ks * KSTEP - g * VEC);
+      wave_lds_fence();
     }
     // Barriers that wait for this wave's LDS accesses only: a fence on the
     // LDS would also wait for the tile, which is on its way there.

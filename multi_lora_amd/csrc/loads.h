@@ -107,6 +107,15 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Between one lane's LDS store and another lane's load of it, in one wave (and
+// between that load and the next store there).  The hardware runs a wave's LDS
+// accesses in order; this keeps the compiler from moving them across, and
+// costs no instruction.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Exclusive prefix sum of `v` over a workgroup of NW wave64s; `*total` gets
 // the sum.  `tmp` is NW ints of LDS.  Every thread of the workgroup must call
 // it.  Loads the caller has in flight are not waited for.

@@ -116,6 +116,7 @@ __device__ __forceinline__ void wide_tile(const ShrinkArgs& a, const TileRef& tr
 #pragma unroll
     for (int u = 0; u < D; ++u) {
       if ((q + u) * kWideWaves + wave >= npieces) break;
+      wave_lds_fence();  // the last piece's fragments are read
       // LDS row r of a block holds source chunk c ^ (r >> 1 & 7) at chunk c.
 #pragma unroll
       for (int b = 0; b < BLOCKS; ++b)
@@ -124,6 +125,7 @@ __device__ __forceinline__ void wide_tile(const ShrinkArgs& a, const TileRef& tr
           const int r = 8 * i + r8;
           *reinterpret_cast<u32x4*>(mine + b * 2048 + r * 128 + ((c8 ^ ((r >> 1) & 7)) << 4)) = v[u][b][i];
         }
+      wave_lds_fence();
       __builtin_amdgcn_sched_barrier(0);
       load(u, q + u + D);
       __builtin_amdgcn_sched_barrier(0);
@@ -143,6 +145,7 @@ __device__ __forceinline__ void wide_tile(const ShrinkArgs& a, const TileRef& tr
   constexpr int UNITS = NB * kWave;
   static_assert(UNITS * sizeof(f32x4) <= BLOCKS * 2048, "a wave's sums fit its part");
   auto red = [&](int w) { return reinterpret_cast<f32x4*>(lds + w * (BLOCKS * 2048)); };
+  wave_lds_fence();
 #pragma unroll
   for (int j = 0; j < NB; ++j) red(wave)[j * kWave + lane] = acc[j];
   __syncthreads();
