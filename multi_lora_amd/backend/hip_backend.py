@@ -76,7 +76,11 @@ class HipLoRABackend(LoRABackend):
 
         Slice ``s`` uses ``a_stacks[s]`` / ``b_stacks[s]`` and writes columns
         ``[col_offsets[s], col_offsets[s] + out_s)`` (default: consecutive).
-        Equal to ``apply_lora`` per slice on the column views, element for element.
+        Decode-shaped batches (no segment over 16 rows, on the slot-grouped
+        path) get ``apply_lora``'s result per slice on the column views,
+        element for element.  For longer segments the order in which the
+        rank-r sums are added is planned for the call's slices together, so
+        the two may differ in the rounding of ``mid``.
         """
         meta = self._meta()
         # The ordinary call, checked and launched natively; what it does not

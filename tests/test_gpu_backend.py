@@ -12,7 +12,8 @@ import torch
 import torch.nn as nn
 
 from multi_lora_amd import AdapterWeights, HipLoRABackend, LinearWithLoRA, MultiLoRAManager, fuse_qkv_projections
-from multi_lora_amd import synthetic
+from multi_lora_amd import _ffi, synthetic
+from multi_lora_amd.synthetic import make_meta
 from oracle.lora_ref import TorchLoRABackend, apply_f64, lora_delta
 from tests.gpu_helpers import assert_tol_f64
 
@@ -51,6 +52,30 @@ def test_apply_lora_multi_equals_per_slice_bitwise(dev):
         hip.apply_lora(wl.x, a, b, sep[:, c0:c0 + b.shape[1]])
     torch.cuda.synchronize()
     assert torch.equal(fused, sep)
+
+
+def test_apply_lora_multi_of_prompts_matches_per_slice(dev):
+    """One prompt of 203 rows at rank 16: q alone runs its whole K in one
+    workgroup, q|k|v splits K.  Both are the same sums, rounded once to mid."""
+    lens, slots, ranks, outs, in_dim = [203], [1], [0, 16], [1024, 256, 256], 4096
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(203, in_dim, generator=g).bfloat16()
+    a = [(torch.randn(2, 16, in_dim, generator=g) * in_dim ** -0.5).bfloat16() for _ in outs]
+    b = [(torch.randn(2, o, 16, generator=g) * 0.05).bfloat16() for o in outs]
+    base, cols = torch.randn(203, sum(outs), generator=g).bfloat16(), [0, 1024, 1280]
+    lib = _ffi.lib()
+    need = [lib.mlora_shrink_workspace_bytes(in_dim, 16, n, 203, 1, 203, _ffi.MLORA_BF16) for n in (1, 3)]
+    assert need[0] == 0 < need[1]                      # the two plans differ
+    hip = HipLoRABackend()
+    hip.set_kernel_input_metadata(make_meta(lens, slots, ranks, [0.0, 1.5], dev, torch.bfloat16))
+    xd, ad, bd = x.to(dev), [t.to(dev) for t in a], [t.to(dev) for t in b]
+    fused, sep = base.to(dev), base.to(dev)
+    hip.apply_lora_multi(xd, ad, bd, fused, cols)
+    for i, c0 in enumerate(cols):
+        hip.apply_lora(xd, ad[i], bd[i], sep[:, c0:c0 + outs[i]])
+    want = apply_f64(x, a, b, make_meta(lens, slots, ranks, [0.0, 1.5], "cpu", torch.bfloat16), base, cols)
+    assert_tol_f64(fused.cpu(), want, "fused")
+    assert_tol_f64(sep.cpu(), want, "per slice")
 
 
 class ToyLM(nn.Module):
