@@ -59,6 +59,20 @@ def test_unaligned_rows(dev, in_dim, pad, dtype):
     run(dev, in_dim, 2, 12, dtype, pad=pad)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("in_dim", [4101, 2111])
+@pytest.mark.parametrize("n_slices,r_max,ranks", [(1, 16, [16, 5, 0, 12]), (2, 16, [16, 5, 0, 12]),
+                                                  (2, 32, [32, 17, 0, 9]), (4, 32, [32, 20, 0, 30])])
+def test_unaligned_long_k(dev, in_dim, n_slices, r_max, ranks, dtype):
+    # Long enough for every wave to load pieces again, by block count.
+    run(dev, in_dim, n_slices, r_max, dtype, ranks=ranks)
+
+
+@pytest.mark.parametrize("in_dim,r_max", [(4100, 16), (2052, 48)])
+def test_fp32_long_k(dev, in_dim, r_max):
+    run(dev, in_dim, 1, r_max, torch.float32, ranks=[r_max, 5, 0, 12])
+
+
 def test_many_one_row_segments_in_fp32(dev):
     run(dev, 520, 2, 16, torch.float32, ranks=[16, 8, 0, 3], lens=[1] * 150, slots=[i % 4 for i in range(150)])
 
