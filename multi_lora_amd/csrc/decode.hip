@@ -756,7 +756,8 @@ __global__ __launch_bounds__(256, (NBT >= 4 && SCHED == kGroupLinked && RS == 2)
   if (j < n_ent) {
     if (shrink) {
       if constexpr (SCHED != kGroupExpandOnly)
-        shrink_items<T, NBT, SCHED, false>(plan, a, j, item, n_ent, en, rows_raw[0], reinterpret_cast<f32x4*>(area), nullptr);
+        shrink_items<T, NBT, SCHED, false>(plan, a, j, item, n_ent, en, rows_raw[0], reinterpret_cast<f32x4*>(area),
+                                           nullptr);
     } else if constexpr (SCHED != kGroupShrinkOnly) {
       expand_items<T, NBT, WN, RS, SCHED, false, ROWB>(plan, a, j, item - n_shrink, n_ent, en, rows_raw,
                                           *reinterpret_cast<DecodeLds<T, WN>*>(area), n_shrink == 0);
@@ -829,11 +830,11 @@ hipError_t launch_dtype(const int32_t* plan, const DecodeArgs& a, const Orders& 
 // ------------------------------------------- fused RMSNorm + decode shrink
 // Shrink launch: grid (e_grid, norm rows + n_shrink), or with ITEM_FAST
 // (n_shrink, norm rows + e_grid).  The first n_norm rows of the grid are
-// RMSNorm row blocks in turn (256 / tpr rows each), written as the RMSNorm kernel writes it, with each row's rstd stored; the
-// items after them are the shrink items of the two-launch schedule, with
-// round(x * w) on the MFMA.  The norm rows come first in the grid, so they
-// run beside the first shrink items instead of after the last.  Nothing in
-// the launch waits on another workgroup.
+// RMSNorm row blocks in turn (256 / tpr rows each), written as the RMSNorm
+// kernel writes them, with each row's rstd stored; the items after them are the
+// shrink items of the two-launch schedule, with round(x * w) on the MFMA.  The
+// norm rows come first, so they run beside the first shrink items instead of
+// after the last.  Nothing in the launch waits on another workgroup.
 template <class T, int NBT, bool ITEM_FAST>
 __global__ __launch_bounds__(256, 4) void planned_norm_shrink_kernel(const int32_t* __restrict__ plan,
                                                                                      int plan_cap, int n_norm,
@@ -953,8 +954,8 @@ hipError_t launch_norm_expand(const int32_t* plan, const DecodeArgs& a, const fl
 }
 
 template <class T>
-hipError_t launch_norm_t(const int32_t* plan, const DecodeArgs& a, const Orders& ord, const NormShrinkArgs& na, int nbt, int phases,
-                         hipStream_t stream) {
+hipError_t launch_norm_t(const int32_t* plan, const DecodeArgs& a, const Orders& ord, const NormShrinkArgs& na, int nbt,
+                         int phases, hipStream_t stream) {
   if (phases & 1) {
     hipError_t e;
     switch (nbt) {
@@ -1178,7 +1179,7 @@ hipError_t launch_build_plan(const SegView& m, int rows, int32_t* plan, int cap,
   return hipGetLastError();
 }
 
-// Which instances a call's two launches run (us, start of the line / with it):
+// Which instances a call's two launches run (us, the other form / this one):
 //   shrink, an entry's items next to each other, past kDirectBlocks A blocks
 //     of items: q|k|v of 256 rows over 112 adapters at rank 32 23.6 / 20.3, at
 //     rank 64 38.1 / 36.2; down of 128 rows over 128 adapters at rank 64 57.8 /
