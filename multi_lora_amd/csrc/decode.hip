@@ -1185,9 +1185,15 @@ hipError_t launch_build_plan(const SegView& m, int rows, int32_t* plan, int cap,
 //     rank 64 38.1 / 36.2; down of 128 rows over 128 adapters at rank 64 57.8 /
 //     48.0.  Smaller grids keep an entry on one XCD (1.00-1.03 of their time
 //     otherwise).
-//   expand, the same order, from 56 column tiles or 40 in a grid of 2048 items,
-//     r_max over 16: gate|up of 77 rows over 40 adapters in r_max 64 36.2 / 33.6;
-//     narrower outputs 1.02-1.2 of their time, r_max 16 the same either way.
+//   expand, the same order, from 32 column tiles in a grid of 2048 items, or
+//     from 56 at r_max over 16.  With the entries fastest an entry's tiles all
+//     run on one XCD, which an entry of many rows among short ones holds up: two
+//     slices of 4544 columns for 257 tokens and segments of 16 and 9 over 122
+//     adapters of ranks 8 and 16 23.4 / 21.2, gate|up for 100 tokens and segments
+//     of 16, 9 and 5 over 90 in r_max 64 91.8 / 76.0.  Even entries at r_max 16
+//     0.97-1.02 of their time, over that 0.85-1.02 (gate|up of 77 rows over 40
+//     adapters in r_max 64 36.2 / 33.6); 24 tiles of even entries up to 1.04, so
+//     they keep the entry order.
 //   expand, B in row order through LDS, past 2048 items at r_max over 32: the same
 //     gate|up 33.6 / 31.5, q|k|v of 128 rows over 128 adapters 24.5 / 23.5;
 //     smaller grids 1.00-1.06 of their time.
@@ -1197,7 +1203,7 @@ static Orders orders_of(const DecodeArgs& a, int nbt) {
   const bool y_fits = a.e_grid <= 65535;  // entries along y
   Orders o;
   o.shrink_fast = y_fits && shrink_items * nbt > kDirectBlocks;
-  o.expand_fast = y_fits && a.r_max > 16 && (a.n_tiles >= 56 || (a.n_tiles >= 40 && expand_items > 2048));
+  o.expand_fast = y_fits && ((a.n_tiles >= 56 && a.r_max > 16) || (a.n_tiles >= 32 && expand_items > 2048));
   o.row_b = a.r_max > 32 && expand_items > 2048;
   return o;
 }

@@ -559,6 +559,7 @@ def test_largest_supported_shape(dev):
     (1032, 14344, 64, [64, 16, 48], 40),      # wide: expand items next to each other, B in row order
     (520, 14344, 32, [32, 7], 40),            # the same with one K-step of B
     (520, 10248, 48, [33, 48], 56),           # 41 column tiles
+    (520, 8968, 16, [16, 7], 72),             # 36 column tiles at r_max 16
 ])
 def test_large_two_launch_grids_equal_the_single_launch(dev, in_dim, out, r_max, ranks, n_slots):
     """Large grids of the two launches (an entry's items next to each other in
